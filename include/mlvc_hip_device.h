@@ -105,7 +105,7 @@ typedef struct mlvc_hip_conv_desc {
     void* y;
     int out_d2s_block;
     int variant;                       /* tile configuration; set by mlvc_hip_conv_plan */
-    int vector_io;                     /* 16-byte row staging eligible; set by mlvc_hip_conv_plan */
+    int vector_io;                     /* row staging (16-byte segments, any width) eligible; set by mlvc_hip_conv_plan */
     int ksplit, split_c;               /* split K; set by mlvc_hip_conv_plan (below) */
     void* workspace;                   /* FP32 partials of a split conv, mlvc_hip_conv_workspace_bytes */
     size_t workspace_bytes;

@@ -220,6 +220,17 @@ void split_rule(const mlvc_hip_conv_desc& d, int& ksplit, int& split_c)
     }
 }
 
+// A channel concat: the second input's pointer, or, in a descriptor planned
+// before its tensors have addresses, the split alone.
+bool concat(const mlvc_hip_conv_desc& d) { return d.x2 || d.ic_split > 0; }
+
+// The input's fusions leave its rows stageable as 16-byte segments: a plain
+// input, or a channel concat whose split falls on 8 channels.
+bool row_staged(const mlvc_hip_conv_desc& d)
+{
+    return d.in_s2d_block <= 1 && d.ic_split % 8 == 0;
+}
+
 bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
 {
     if (k.bm == 0 || k.kh != d.kh || k.kw != d.kw || k.s != d.stride_h || k.s != d.stride_w) return false;
@@ -233,10 +244,10 @@ bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
     if (d.epilogue == MLVC_EPI_REGLU && k.bm % 64 != 0) return false;
     if (d.kh == 1 && (d.pad_h || d.pad_w)) return false;
     // The weight-streaming kernel: plain NCHW input staged as 16-byte rows,
-    // no ReGLU, DEPTH_TO_SPACE(2) or none, 8-aligned output rows.
-    if (k.ws_ic && (d.x2 || d.in_s2d_block > 1 || d.epilogue == MLVC_EPI_REGLU || d.out_d2s_block > 2 ||
-                    d.iw % 8 != 0 || d.ow % 8 != 0))
-        return false;
+    // no ReGLU, DEPTH_TO_SPACE(2) or none; rows of a multiple of 8 pixels in
+    // and out, or of any width where the variant has ragged builds (NCHW).
+    if (k.ws_ic && (concat(d) || d.in_s2d_block > 1 || d.epilogue == MLVC_EPI_REGLU || d.out_d2s_block > 2)) return false;
+    if (k.ws_ic && (d.iw % 8 != 0 || d.ow % 8 != 0) && (!k.launch_rag[0] || d.in_nhwc || d.out_nhwc)) return false;
     int ih, iw, oh, ow;
     kernel_geometry(d, ih, iw, oh, ow);
     // ...and its 16-byte row staging keeps buffer offsets (up to KC channel
@@ -272,7 +283,12 @@ int mlvc_hip_conv_plan(mlvc_hip_conv_desc* desc)
                                ((d.oc + k.bm - 1) / k.bm) * d.n;
             const long rounds = (tiles + slots - 1) / slots;
             // Work per round in MACs plus a fixed per-tile overhead.
-            const double cost = static_cast<double>(rounds) * (static_cast<double>(k.bm) * k.th * k.tw + 4096.0);
+            double cost = static_cast<double>(rounds) * (static_cast<double>(k.bm) * k.th * k.tw + 4096.0);
+            // Ragged rows without the ragged builds are staged pixel by pixel,
+            // 16 or 32 two-byte loads each: 3 to 12 times the time of the row
+            // staging over 3x3 convs of 27 to 369 pixels wide (256->256 stride 2
+            // on 58x103: 213 us against 18 us; 64->64 on 127x226: 27 against 9).
+            if (row_staged(d) && !k.launch_rag[0] && (iw % 8 != 0 || (k.ws_ic && ow % 8 != 0))) cost *= 8.0;
             if (best == 0 || cost < best_cost) {
                 best = v;
                 best_cost = cost;
@@ -283,9 +299,7 @@ int mlvc_hip_conv_plan(mlvc_hip_conv_desc* desc)
             desc->ksplit = 1;
             desc->split_c = d.ic;
         }
-        // 16-byte row-segment staging: plain or channel-concat input whose
-        // split falls on 8 channels, rows of 8-aligned width.
-        desc->vector_io = best != 0 && d.in_s2d_block <= 1 && (!d.x2 || d.ic_split % 8 == 0) && iw % 8 == 0;
+        desc->vector_io = best != 0 && row_staged(d);
     });
 }
 
@@ -430,8 +444,17 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             // Buffer offsets of the vector path stay below 2^31 (range check
             // and the out-of-range marker); the concat split falls on a chunk.
             const std::uint64_t plane_bytes = static_cast<std::uint64_t>(a.ih) * a.iw * 2;
-            const bool vec = d.vector_io && aligned && a.s2d <= 1 && (!a.x2 || a.ic_split % k.kc == 0) &&
-                             a.iw % 8 == 0 && (static_cast<std::uint64_t>(d.ic) + k.kc) * plane_bytes < (1ull << 31);
+            const bool rows = d.vector_io && aligned && a.s2d <= 1 && (!a.x2 || a.ic_split % k.kc == 0) &&
+                              (static_cast<std::uint64_t>(d.ic) + k.kc) * plane_bytes < (1ull << 31);
+            // Rows of a multiple of 8 pixels (for the weight-streaming kernel,
+            // output rows too); else the ragged builds, whose buffer loads
+            // need every image's first element on 4 bytes.
+            const bool even = a.iw % 8 == 0 && (!k.ws_ic || a.ow % 8 == 0);
+            const std::uint64_t plane = static_cast<std::uint64_t>(a.ih) * a.iw;
+            const bool images4 = d.n == 1 || ((a.x2 ? a.ic_split : d.ic) * plane % 2 == 0 &&
+                                              (!a.x2 || (d.ic - a.ic_split) * plane % 2 == 0));
+            const bool vec = rows && even;
+            const auto ragged = rows && !even && images4 ? k.launch_rag[a.iw & 1] : nullptr;
             a.tiles_x = (a.ow + k.tw - 1) / k.tw;
             a.nchunks = (d.ic + k.kc - 1) / k.kc;
             a.tiles = a.tiles_x * ((a.oh + k.th - 1) / k.th);
@@ -445,8 +468,9 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             const std::uint64_t src_plane = static_cast<std::uint64_t>(a.ih) * a.iw * 4 * 2;
             const bool s2d_vec = k.launch_s2d && a.s2d == 2 && (reinterpret_cast<std::uintptr_t>(d.x) & 15u) == 0 &&
                                  a.iw % 8 == 0 && (static_cast<std::uint64_t>(d.ic / 4) + k.kc / 4 + 1) * src_plane < (1ull << 31);
-            if (k.ws_ic && !vec) throw std::runtime_error("conv: variant needs 16-byte row staging");
-            (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : k.launch_scalar)(a, grid, to_stream(s));
+            if (k.ws_ic && (d.x2 || a.s2d > 1)) throw std::runtime_error("conv: variant needs a plain input");
+            if (k.ws_ic && !vec && (even || !k.launch_scalar)) throw std::runtime_error("conv: variant needs 16-byte row staging");
+            (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : ragged ? ragged : k.launch_scalar)(a, grid, to_stream(s));
             if (a.ksplit > 1) {
                 ConvArgs r = a;  // the reduce works in the real output geometry
                 r.ih = d.ih;

@@ -7,10 +7,10 @@ namespace conv {
 
 namespace {
 const Variant kTable[] = {
-    MLVC_VARIANT(32, 1, 256, 1, 1, 1, 32),
-    MLVC_VARIANT(64, 1, 256, 1, 1, 1, 32),
-    MLVC_VARIANT(64, 1, 128, 1, 1, 1, 32),
-    MLVC_VARIANT(128, 1, 128, 1, 1, 1, 32),
+    with_ragged<32, 1, 256, 1, 1, 1, 32>(MLVC_VARIANT(32, 1, 256, 1, 1, 1, 32)),
+    with_ragged<64, 1, 256, 1, 1, 1, 32>(MLVC_VARIANT(64, 1, 256, 1, 1, 1, 32)),
+    with_ragged<64, 1, 128, 1, 1, 1, 32>(MLVC_VARIANT(64, 1, 128, 1, 1, 1, 32)),
+    with_ragged<128, 1, 128, 1, 1, 1, 32>(MLVC_VARIANT(128, 1, 128, 1, 1, 1, 32)),
     MLVC_VARIANT_S2D(64, 2, 64, 1, 1, 1, 32),
     MLVC_VARIANT_S2D(64, 4, 32, 1, 1, 1, 32),
 };

@@ -8,8 +8,8 @@ namespace conv {
 namespace {
 const Variant kTable[] = {
     MLVC_VARIANT_OCC(32, 4, 64, 3, 3, 1, 16, 4),
-    MLVC_VARIANT_OCC(32, 8, 32, 3, 3, 1, 16, 4),
-    MLVC_VARIANT_OCC(64, 4, 32, 3, 3, 1, 16, 4),
+    with_ragged<32, 8, 32, 3, 3, 1, 16, 1, 4, 4>(MLVC_VARIANT_OCC(32, 8, 32, 3, 3, 1, 16, 4)),
+    with_ragged<64, 4, 32, 3, 3, 1, 16, 1, 4, 4>(MLVC_VARIANT_OCC(64, 4, 32, 3, 3, 1, 16, 4)),
     MLVC_VARIANT_S2D(32, 4, 64, 3, 3, 1, 16),
     MLVC_VARIANT_S2D(32, 8, 32, 3, 3, 1, 16),
     MLVC_VARIANT_S2D(64, 4, 64, 3, 3, 1, 16),
@@ -37,18 +37,18 @@ const Variant kTable[] = {
     MLVC_VARIANT_DB(128, 4, 64, 3, 3, 1, 16),
     MLVC_VARIANT_DB(64, 4, 64, 3, 3, 1, 16),
     MLVC_VARIANT_OCC(32, 2, 64, 3, 3, 1, 16, 4),
-    MLVC_VARIANT_WO(32, 2, 32, 3, 3, 1, 16, 1, 2, 4),
+    with_ragged<32, 2, 32, 3, 3, 1, 16, 1, 2, 4>(MLVC_VARIANT_WO(32, 2, 32, 3, 3, 1, 16, 1, 2, 4)),
     MLVC_VARIANT_WO(64, 2, 32, 3, 3, 1, 16, 1, 2, 4),
     MLVC_VARIANT_WS(256, 4, 32, 128, 2),
     MLVC_VARIANT_WS(128, 4, 32, 128, 2),
-    MLVC_VARIANT_WS(256, 4, 32, 64, 2),
-    MLVC_VARIANT_WS(128, 4, 32, 64, 2),
-    MLVC_VARIANT_WS(256, 2, 32, 128, 2),
+    with_ragged_ws<WsCfg<256, 4, 32, 64, 2>>(MLVC_VARIANT_WS(256, 4, 32, 64, 2)),
+    with_ragged_ws<WsCfg<128, 4, 32, 64, 2>>(MLVC_VARIANT_WS(128, 4, 32, 64, 2)),
+    with_ragged_ws<WsCfg<256, 2, 32, 128, 2>>(MLVC_VARIANT_WS(256, 2, 32, 128, 2)),
     MLVC_VARIANT_WSR(128, 4, 32, 64, 2, 9),
     MLVC_VARIANT_WSR(256, 2, 32, 128, 2, 9),
     // Widths that divide 120 and 240 (24, 40) or 240 and 480 (48), so the
     // 68x120 and 136x240 decoder convs run without padded columns.
-    MLVC_VARIANT_WSR(128, 4, 24, 64, 2, 9),
+    with_ragged_ws<WsCfg<128, 4, 24, 64, 2, 1, 4, 9>>(MLVC_VARIANT_WSR(128, 4, 24, 64, 2, 9)),
     MLVC_VARIANT_WSR(128, 8, 24, 64, 2, 9),
     MLVC_VARIANT_WSR(128, 4, 40, 64, 2, 9),
     MLVC_VARIANT_WSR(128, 4, 48, 64, 2, 9),
@@ -63,13 +63,13 @@ const Variant kTable[] = {
     MLVC_VARIANT_WSP(128, 4, 48, 32, 2, 9),
     MLVC_VARIANT_WSP(128, 4, 24, 32, 2, 9),
     // 64 output channels on two waves, more workgroups per CU.
-    MLVC_VARIANT_WSW(64, 2, 32, 64, 4, 2, 9),
+    with_ragged_ws<WsCfg<64, 2, 32, 64, 4, 1, 2, 9>>(MLVC_VARIANT_WSW(64, 2, 32, 64, 4, 2, 9)),
     MLVC_VARIANT_WSW(64, 4, 32, 64, 3, 2, 9),
     MLVC_VARIANT_WSW(64, 8, 32, 64, 2, 2, 9),
     // Short, narrow tiles: enough workgroups for deep convs over few pixels
     // (46x80 and 92x160 planes).
-    MLVC_VARIANT_WSW(64, 2, 16, 64, 4, 2, 9),
-    MLVC_VARIANT_WSR(128, 2, 16, 64, 2, 9),
+    with_ragged_ws<WsCfg<64, 2, 16, 64, 4, 1, 2, 9>>(MLVC_VARIANT_WSW(64, 2, 16, 64, 4, 2, 9)),
+    with_ragged_ws<WsCfg<128, 2, 16, 64, 2, 1, 4, 9>>(MLVC_VARIANT_WSR(128, 2, 16, 64, 2, 9)),
     // 512 output channels at 136x240 in one round of two workgroups per CU:
     // 255 8x16 tiles x 2 channel blocks = 510 workgroups, where the 4x48
     // tiles' 680 take two rounds of 512 slots with the second a third full.

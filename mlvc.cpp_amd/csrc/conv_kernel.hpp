@@ -184,6 +184,90 @@ __device__ __forceinline__ std::uint16_t reglu_h(std::uint16_t g, std::uint16_t 
     return f2h(mul_f32(h2f(f2h(c)), h2f(l)));
 }
 
+// Eight pixels of an input row of any width, read with dword-aligned buffer
+// loads. RAG 1: the row starts on 4 bytes, one 16-byte load (a buffer load
+// needs dword alignment only, and its range check works dword by dword). RAG
+// 2 (odd widths): the row may start 2 bytes past a dword, so the 16 bytes
+// from the dword below and the next dword are loaded and shifted by a half.
+template <int RAG>
+struct RaggedRow {
+    u32x4 v;
+};
+template <>
+struct RaggedRow<2> {
+    u32x4 v;
+    std::uint32_t next;
+};
+
+template <int RAG>
+__device__ __forceinline__ RaggedRow<RAG> ragged_load(__amdgpu_buffer_rsrc_t r, std::uint32_t off)
+{
+    RaggedRow<RAG> row;
+    const std::uint32_t at = RAG == 2 ? off & ~3u : off;
+    row.v = __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(at), 0, 0);
+    if constexpr (RAG == 2) row.next = __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(at + 16u), 0, 0);
+    return row;
+}
+
+// The eight pixels; bit 0 of `parity` says whether the row started in the
+// upper half of its first dword (the element offset's lowest bit: for 8
+// channels from an even one at an even column of odd-width rows, that of
+// channel * ih + row).
+template <int RAG>
+__device__ __forceinline__ u32x4 ragged_row(const RaggedRow<RAG>& row, int parity)
+{
+    if constexpr (RAG != 2) {
+        return row.v;
+    } else {
+        const std::uint32_t sh = (parity & 1) * 16;
+        return u32x4{__builtin_amdgcn_alignbit(row.v[1], row.v[0], sh), __builtin_amdgcn_alignbit(row.v[2], row.v[1], sh),
+                     __builtin_amdgcn_alignbit(row.v[3], row.v[2], sh), __builtin_amdgcn_alignbit(row.next, row.v[3], sh)};
+    }
+}
+
+// Eight halves at any element address (16-byte accesses on 2 bytes are legal
+// on gfx950; the type keeps the compiler from assuming more).
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+
+// Plain NCHW epilogue of eight rounded outputs h of one row, at element
+// offset o of y (and of the residual); V is the access type.
+template <class V>
+__device__ __forceinline__ void store_row8(const ConvArgs& a, u32x4 h, size_t o, bool max_form)
+{
+    if (a.epi == MLVC_EPI_LEAKY_RELU) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) h[k] = leaky_h2(h[k], a.alpha, max_form);
+    } else if (a.epi == MLVC_EPI_CLAMP) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) h[k] = clamp_h2(h[k], a.lo, a.hi);
+    } else if (a.epi == MLVC_EPI_RESIDUAL_ADD) {
+        const u32x4 r = *reinterpret_cast<const V*>(a.res + o);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            h[k] = f2h(lo_f16(h[k]) + lo_f16(r[k])) | (static_cast<std::uint32_t>(f2h(hi_f16(h[k]) + hi_f16(r[k]))) << 16);
+    }
+    *reinterpret_cast<V*>(a.y + o) = h;
+}
+
+// The first `n` of them (a row's last, partial group).
+__device__ __forceinline__ void store_row_part(const ConvArgs& a, u32x4 h8, size_t o, int n)
+{
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (j >= n) continue;
+        std::uint16_t h = static_cast<std::uint16_t>(h8[j >> 1] >> (16 * (j & 1)));
+        if (a.epi == MLVC_EPI_LEAKY_RELU) {
+            const float f = h2f(h);
+            if (f < 0.0f) h = leaky_f16(f, a.alpha);
+        } else if (a.epi == MLVC_EPI_CLAMP) {
+            h = clamp_h(h, a.lo, a.hi);
+        } else if (a.epi == MLVC_EPI_RESIDUAL_ADD) {
+            h = f2h(h2f(h) + h2f(a.res[o + j]));
+        }
+        a.y[o + j] = h;
+    }
+}
+
 template <int BM_, int TH_, int TW_, int KH_, int KW_, int S_, int KC_, int STG_, bool DB_, int WM_ = 1, int WNW_ = 4,
           int OCC_ = 2>
 struct Cfg {
@@ -191,10 +275,13 @@ struct Cfg {
     // Input staging: 0 = per-pixel loads through the SPACE_TO_DEPTH / CONCAT
     // maps; 1 = 16-byte row segments of 8 channels, transposed in registers;
     // 2 = 16-byte source-row segments through SPACE_TO_DEPTH(2) (each dword
-    // already holds the dx = 0, 1 channel pair of one staged pixel).
+    // already holds the dx = 0, 1 channel pair of one staged pixel). 3 and 4
+    // are 1 for rows of any even and any odd number of pixels (RaggedRow).
     // 1 and 2 need W % 8 == 0.
     static constexpr int STG = STG_;
     static constexpr bool VEC = STG_ != 0;
+    static constexpr int RAG = STG_ >= 3 ? STG_ - 2 : 0;
+    static constexpr bool ROWS = STG_ == 1 || RAG != 0;  // row segments transposed in registers
     // Two LDS stages: chunk k+1 is staged (weights by LDS DMA) while chunk k
     // is multiplied, one barrier per chunk. Otherwise one stage, weights
     // staged through registers, two barriers per chunk, half the LDS.
@@ -294,7 +381,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
 
     const size_t hw = static_cast<size_t>(a.ih) * a.iw;
     const int c1 = a.x2 ? a.ic_split : a.ic;
-    u32x4 vin[C::STG == 1 ? C::UNITS_PER_T : 1][8];
+    RaggedRow<C::RAG> vin[C::ROWS ? C::UNITS_PER_T : 1][8];
     u32x4 vs2[C::STG == 2 ? C::UNITS2_PER_T : 1][C::STG == 2 ? C::KC / 4 : 1][2][2];
     std::uint32_t in_reg[C::VEC ? 1 : C::PIX_PER_T][C::KC / 2];
     u32x4 w_reg[C::DB ? 1 : C::W_PER_T];
@@ -306,12 +393,13 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
     const std::uint32_t hw2 = static_cast<std::uint32_t>(hw) * 2u;
     const std::uint16_t* x_img = a.x + static_cast<size_t>(b) * c1 * hw;
     const std::uint16_t* x2_img = a.x2 ? a.x2 + static_cast<size_t>(b) * (a.ic - c1) * hw : x_img;
+    const auto whole = [](std::uint32_t bytes) { return static_cast<int>(C::RAG ? (bytes + 3u) & ~3u : bytes); };
     const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<std::uint16_t*>(x_img), 0, static_cast<int>(c1 * hw2), kRawBufferFlags);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<std::uint16_t*>(x_img), 0, whole(c1 * hw2), kRawBufferFlags);
     const __amdgpu_buffer_rsrc_t rx2 = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<std::uint16_t*>(x2_img), 0, static_cast<int>(a.x2 ? (a.ic - c1) * hw2 : 0u), kRawBufferFlags);
-    std::uint32_t pix_off[C::STG == 1 ? C::UNITS_PER_T : 1];
-    int unit_c8[C::STG == 1 ? C::UNITS_PER_T : 1];
+        const_cast<std::uint16_t*>(x2_img), 0, whole(a.x2 ? (a.ic - c1) * hw2 : 0u), kRawBufferFlags);
+    std::uint32_t pix_off[C::ROWS ? C::UNITS_PER_T : 1];
+    int unit_c8[C::ROWS ? C::UNITS_PER_T : 1];
     // STG 2: the source image is [IC/4][2*IH][2*IW]; staged pixel (iy, ix)
     // channel 4*cs + 2*dy + dx is source (cs, 2*iy + dy, 2*ix + dx).
     const int sw2 = a.iw * 2, sh2 = a.ih * 2;
@@ -330,7 +418,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
             src_off[i] = ok ? static_cast<std::uint32_t>(2 * iy * sw2 + 2 * ix) * 2u : kOutOfRange;
         }
     }
-    if constexpr (C::STG == 1) {
+    if constexpr (C::ROWS) {
 #pragma unroll
         for (int i = 0; i < C::UNITS_PER_T; ++i) {
             const int u = tid + i * C::kThreads;
@@ -362,7 +450,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
                                     : src_off[i] + (cs0 + q) * splane2 + static_cast<std::uint32_t>(dy * sw2 * 2 + hh * 16);
                             vs2[i][q][dy][hh] = __builtin_amdgcn_raw_buffer_load_b128(rs, static_cast<int>(off), 0, 0);
                         }
-        } else if constexpr (C::STG == 1) {
+        } else if constexpr (C::ROWS) {
             const bool second = a.x2 && c0 >= c1;
             const __amdgpu_buffer_rsrc_t r = second ? rx2 : rx;
             const std::uint32_t cbase = static_cast<std::uint32_t>(second ? c0 - c1 : c0);
@@ -374,8 +462,14 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
                 // The channel offset goes in the VGPR operand: the range check
                 // covers that operand only, so channels past the end read zeros.
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    vin[i][k] = __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off + k * hw2), 0, 0);
+                for (int k = 0; k < 8; ++k) {
+                    std::uint32_t at = off + k * hw2;
+                    if constexpr (C::RAG != 0) {  // rounded-up resources: channels past the end are named, not range-checked
+                        const int cn = second ? a.ic - c1 : c1;
+                        if (off == kOutOfRange || static_cast<int>(cbase) + unit_c8[i] * 8 + k >= cn) at = kOutOfRange;
+                    }
+                    vin[i][k] = ragged_load<C::RAG>(r, at);
+                }
             }
         } else {
 #pragma unroll
@@ -429,7 +523,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
                     }
                 }
             }
-        } else if constexpr (C::STG == 1) {
+        } else if constexpr (C::ROWS) {
             // 8x8 transpose in registers: staged pixel j of the segment gets
             // the 8 channels of the unit as one 16-byte LDS write.
 #pragma unroll
@@ -437,12 +531,19 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
                 const int u = tid + i * C::kThreads;
                 if (u < C::UNITS) {
                     const int sg = u % C::NSEG, yi = (u / C::NSEG) % C::IH_T, c8 = u / (C::NSEG * C::IH_T);
+                    u32x4 v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = ragged_row<C::RAG>(vin[i][k], (k & a.ih) + iy0 + yi);
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
                         const bool up = j & 1;
                         const int wd = j >> 1;
-                        const u32x4 t = {pack_half(vin[i][0][wd], vin[i][1][wd], up), pack_half(vin[i][2][wd], vin[i][3][wd], up),
-                                         pack_half(vin[i][4][wd], vin[i][5][wd], up), pack_half(vin[i][6][wd], vin[i][7][wd], up)};
+                        u32x4 t = {pack_half(v[0][wd], v[1][wd], up), pack_half(v[2][wd], v[3][wd], up),
+                                   pack_half(v[4][wd], v[5][wd], up), pack_half(v[6][wd], v[7][wd], up)};
+                        if constexpr (C::RAG != 0) {
+                            // Columns past the row's end hold the next row: padding reads zeros.
+                            if (xa + sg * 8 + j >= a.iw) t = u32x4{0u, 0u, 0u, 0u};
+                        }
                         *reinterpret_cast<u32x4*>(&in_s[C::at(yi, sg * 8 + j) + c8 * 8]) = t;
                     }
                 }
@@ -664,33 +765,32 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
         return;
     }
 
-    // Stage 2: the epilogue acts on the rounded value. Vector path: 8
-    // consecutive pixels of a channel per thread, 16-byte loads and stores.
-    if (a.ow % 8 == 0 && a.d2s <= 1) {
+    // Stage 2: the epilogue acts on the rounded value, 8 consecutive pixels of
+    // a channel per thread with 16-byte loads and stores. Rows of a ragged
+    // width end in a partial group, stored element by element (before, every
+    // element of such an output left alone as two bytes).
+    if (a.d2s <= 1) {
         constexpr int GROUPS = C::BN / 8;
-        for (int u = tid; u < C::BM * GROUPS; u += C::kThreads) {
+        auto group = [&](int u, auto store) {
             const int g = u % GROUPS, ocl = u / GROUPS, oc = ocb * C::BM + ocl;
             const int pl = g * 8, oy = ty0 + pl / C::TW, ox = tx0 + pl % C::TW;
-            if (oc >= a.oc || oy >= a.oh || ox >= a.ow) continue;
-            u32x4 h = *reinterpret_cast<const u32x4*>(&lds[ocl * C::EPI_ROW + pl]);
-            const size_t o = (static_cast<size_t>(b * a.oc + oc) * a.oh + oy) * a.ow + ox;
-            if (a.epi == MLVC_EPI_LEAKY_RELU) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) h[k] = leaky_h2(h[k], a.alpha, max_form);
-            } else if (a.epi == MLVC_EPI_CLAMP) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) h[k] = clamp_h2(h[k], a.lo, a.hi);
-            } else if (a.epi == MLVC_EPI_RESIDUAL_ADD) {
-                const u32x4 r = *reinterpret_cast<const u32x4*>(a.res + o);
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    h[k] = f2h(lo_f16(h[k]) + lo_f16(r[k])) | (static_cast<std::uint32_t>(f2h(hi_f16(h[k]) + hi_f16(r[k]))) << 16);
-            }
-            *reinterpret_cast<u32x4*>(a.y + o) = h;
+            if (oc >= a.oc || oy >= a.oh || ox >= a.ow) return;
+            const u32x4 h = *reinterpret_cast<const u32x4*>(&lds[ocl * C::EPI_ROW + pl]);
+            store(h, (static_cast<size_t>(b * a.oc + oc) * a.oh + oy) * a.ow + ox, ox);
+        };
+        if (a.ow % 8 == 0) {
+            for (int u = tid; u < C::BM * GROUPS; u += C::kThreads)
+                group(u, [&](u32x4 h, size_t o, int) { store_row8<u32x4>(a, h, o, max_form); });
+        } else {
+            for (int u = tid; u < C::BM * GROUPS; u += C::kThreads)
+                group(u, [&](u32x4 h, size_t o, int ox) {
+                    if (ox + 8 <= a.ow) store_row8<u32x4_any>(a, h, o, max_form);
+                    else store_row_part(a, h, o, a.ow - ox);
+                });
         }
         return;
     }
-    // Element by element (ragged widths, other DEPTH_TO_SPACE blocks).
+    // Element by element (DEPTH_TO_SPACE blocks other than 2).
     for (int e = tid; e < C::BM * C::BN; e += C::kThreads) {
         const int ocl = e / C::BN, pl = e - ocl * C::BN;
         const int oc = ocb * C::BM + ocl;
@@ -722,12 +822,24 @@ struct Variant {
     // Its channel-last output tile fits the LDS: bit 0 plain, bit 1 with
     // DEPTH_TO_SPACE(2).
     int nhwc_out = 0;
+    // Row staging of widths that are no multiple of 8: even, odd (or null:
+    // such widths are staged pixel by pixel, by launch_scalar).
+    void (*launch_rag[2])(const ConvArgs&, dim3, hipStream_t) = {nullptr, nullptr};
 };
 
 template <class C>
 void launch_mfma(const ConvArgs& a, dim3 grid, hipStream_t s)
 {
     hipLaunchKernelGGL(conv_mfma_kernel<C>, grid, dim3(C::kThreads), 0, s, a);
+}
+
+// A one-stage variant with row staging of ragged widths (STG 3 and 4).
+template <int BM, int TH, int TW, int KH, int KW, int S, int KC, int WM = 1, int WNW = 4, int OCC = 2>
+constexpr Variant with_ragged(Variant v)
+{
+    v.launch_rag[0] = &launch_mfma<Cfg<BM, TH, TW, KH, KW, S, KC, 3, false, WM, WNW, OCC>>;
+    v.launch_rag[1] = &launch_mfma<Cfg<BM, TH, TW, KH, KW, S, KC, 4, false, WM, WNW, OCC>>;
+    return v;
 }
 
 #define MLVC_VARIANT(BM, TH, TW, KH, KW, S, KC)                                                              \

@@ -84,7 +84,11 @@ struct WsCfg {
     __device__ static constexpr int at(int row, int x) { return row * ROW + x * PST; }
 };
 
-template <class C>
+// RAG: how input rows are aligned. 0: rows of a multiple of 8 pixels, so every
+// 16-byte segment is aligned and lies inside the row or outside it; 1: rows of
+// an even number of pixels (segments on 4 bytes); 2: rows of an odd number
+// (segments on 2 bytes, RaggedRow). Plain NCHW input only for 1 and 2.
+template <class C, int RAG>
 __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::OCC))) void conv_ws_kernel(ConvArgs a)
 {
     __shared__ __attribute__((aligned(16))) std::uint16_t lds[C::LDS];
@@ -107,8 +111,8 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
     const size_t hw = static_cast<size_t>(a.ih) * a.iw;
     const std::uint32_t hw2 = static_cast<std::uint32_t>(hw) * 2u;
     const std::uint16_t* x_img = a.x + static_cast<size_t>(b) * a.ic * hw;
-    const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<std::uint16_t*>(x_img), 0, static_cast<int>(a.ic * hw2), kRawBufferFlags);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<std::uint16_t*>(x_img), 0, static_cast<int>(RAG == 0 ? a.ic * hw2 : (a.ic * hw2 + 3u) & ~3u), kRawBufferFlags);
     // Unit i of this thread (units i0 .. i0 + N - 1 in v[0 .. N-1]): issue
     // its eight row loads, then write it transposed into the halo buffer at
     // LDS offset boff.
@@ -127,6 +131,15 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
 #pragma unroll
         for (int k = 0; k < 8; ++k) v[k] = load_row(off, k);
     };
+    // Ragged rows: the unit's loads (rv) end in the same eight segments.
+    auto issue_ragged = [&](int cb, int i, RaggedRow<RAG> (&rv)[8]) {
+        const int u = tid + i * C::kThreads;
+        const std::uint32_t off = unit_off(cb, i);
+        const int c0 = cb + u / (C::NSEG * C::IH_T) * 8;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            rv[k] = ragged_load<RAG>(rx, off == kOutOfRange || c0 + k >= a.ic ? kOutOfRange : off + k * hw2);
+    };
     auto put = [&](int i, const u32x4 (&v)[8], int boff) {
         const int u = tid + i * C::kThreads;
         if (i >= C::UNITS_PER_T || u >= C::UNITS) return;
@@ -135,8 +148,12 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
         for (int j = 0; j < 8; ++j) {
             const bool up = j & 1;
             const int wd = j >> 1;
-            const u32x4 t = {pack_half(v[0][wd], v[1][wd], up), pack_half(v[2][wd], v[3][wd], up),
-                             pack_half(v[4][wd], v[5][wd], up), pack_half(v[6][wd], v[7][wd], up)};
+            u32x4 t = {pack_half(v[0][wd], v[1][wd], up), pack_half(v[2][wd], v[3][wd], up),
+                       pack_half(v[4][wd], v[5][wd], up), pack_half(v[6][wd], v[7][wd], up)};
+            if constexpr (RAG != 0) {
+                // Columns past the row's end hold the next row: padding reads zeros.
+                if (xa + sg * 8 + j >= a.iw) t = u32x4{0u, 0u, 0u, 0u};
+            }
             const int col = C::S == 1 ? sg * 8 + j : (j & 1) * C::HALF + sg * 4 + (j >> 1);
             *reinterpret_cast<u32x4*>(&lds[boff + C::at(yi, col) + c8 * 8]) = t;
         }
@@ -159,6 +176,25 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
         *reinterpret_cast<u32x4*>(&lds[boff + C::at(yi, lc) + c8 * 8]) = v;
     };
     auto stage = [&](int cb) {
+        if constexpr (RAG != 0) {
+            static_assert(!C::PIPE, "ragged rows are staged between passes");
+            constexpr int BATCH = C::STAGE_BATCH;
+#pragma unroll
+            for (int i0 = 0; i0 < C::UNITS_PER_T; i0 += BATCH) {
+                RaggedRow<RAG> rv[BATCH][8];
+#pragma unroll
+                for (int ii = 0; ii < BATCH; ++ii) issue_ragged(cb, i0 + ii, rv[ii]);
+#pragma unroll
+                for (int ii = 0; ii < BATCH; ++ii) {
+                    const int yi = ((tid + (i0 + ii) * C::kThreads) / C::NSEG) % C::IH_T;
+                    u32x4 v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = ragged_row<RAG>(rv[ii][k], (k & a.ih) + iy0 + yi);
+                    put(i0 + ii, v, 0);
+                }
+            }
+            return;
+        }
         if (a.in_nhwc) {
             constexpr int PB = 8;  // pieces in flight per thread
 #pragma unroll
@@ -478,33 +514,37 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
         const int g = u % GROUPS, ocl = u / GROUPS, oc = ocb * C::BM + ocl;
         const int pl = g * 8, oy = ty0 + pl / C::TW, ox = tx0 + pl % C::TW;
         if (oc >= a.oc || oy >= a.oh || ox >= a.ow) continue;
-        u32x4 h = *reinterpret_cast<const u32x4*>(&lds[ocl * C::EPI_ROW + pl]);
+        const u32x4 h = *reinterpret_cast<const u32x4*>(&lds[ocl * C::EPI_ROW + pl]);
         const size_t o = (static_cast<size_t>(b * a.oc + oc) * a.oh + oy) * a.ow + ox;
-        if (a.epi == MLVC_EPI_LEAKY_RELU) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) h[k] = leaky_h2(h[k], a.alpha, max_form);
-        } else if (a.epi == MLVC_EPI_CLAMP) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) h[k] = clamp_h2(h[k], a.lo, a.hi);
-        } else if (a.epi == MLVC_EPI_RESIDUAL_ADD) {
-            const u32x4 r = *reinterpret_cast<const u32x4*>(a.res + o);
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                h[k] = f2h(lo_f16(h[k]) + lo_f16(r[k])) | (static_cast<std::uint32_t>(f2h(hi_f16(h[k]) + hi_f16(r[k]))) << 16);
-        }
-        *reinterpret_cast<u32x4*>(a.y + o) = h;
+        if constexpr (RAG == 0) store_row8<u32x4>(a, h, o, max_form);
+        else if (ox + 8 <= a.ow) store_row8<u32x4_any>(a, h, o, max_form);
+        else store_row_part(a, h, o, a.ow - ox);
     }
 }
 
-template <class C>
+template <class C, int RAG = 0>
 void launch_ws(const ConvArgs& a, dim3 grid, hipStream_t s)
 {
-    hipLaunchKernelGGL(conv_ws_kernel<C>, grid, dim3(C::kThreads), 0, s, a);
+    hipLaunchKernelGGL((conv_ws_kernel<C, RAG>), grid, dim3(C::kThreads), 0, s, a);
+}
+
+// A variant that also runs NCHW rows of any width: the ragged builds, and for
+// operands without the alignment those need (x off 16 bytes, images off 4) the
+// per-pixel staging of conv_mfma_kernel on the same tile, whose packed weights
+// are the same.
+template <class C>
+constexpr Variant with_ragged_ws(Variant v)
+{
+    v.launch_scalar = &launch_mfma<Cfg<C::BM, C::TH, C::TW, 3, 3, C::S, 16, 0, false, C::WAVES, 1, 1>>;
+    v.launch_rag[0] = &launch_ws<C, 1>;
+    v.launch_rag[1] = &launch_ws<C, 2>;
+    return v;
 }
 
 // Variant entry: weights packed with kc = 16 ([ocb][c16][tap][m-tile][lane][8]);
 // eligible for plain NCHW inputs with 16-byte rows (the vector launch slot),
-// staged SC channels per pass; no scalar or SPACE_TO_DEPTH staging.
+// staged SC channels per pass; other widths where with_ragged_ws adds them; no
+// SPACE_TO_DEPTH staging.
 #define MLVC_VARIANT_WS(BM, TH, TW, SC, OCC)                                                                   \
     Variant{"ws_bm" #BM "_" #TH "x" #TW "_k3x3_s1_sc" #SC "_occ" #OCC, BM, TH, TW, 3, 3, 1, 16, nullptr,          \
             &launch_ws<WsCfg<BM, TH, TW, SC, OCC>>, nullptr, SC, WsCfg<BM, TH, TW, SC, OCC>::NHWC_OUT}
