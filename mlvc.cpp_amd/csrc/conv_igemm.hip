@@ -1,11 +1,12 @@
 // FP16 convolution (groups == 1): variant table, planning, weight packing
 // and launch behind the device C ABI. The MFMA kernel template is in
 // conv_kernel.hpp and its tile variants are instantiated per kernel size in
-// conv_k3s1.hip, conv_k3s2.hip and conv_k1.hip.
+// conv_k3s1.hip, conv_k3s2.hip and conv_k1.hip (1x1 also in conv_point.hip).
 
 #include "conv_kernel.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -17,6 +18,7 @@ namespace conv {
 const Variant* variants_k3s1(int* n);
 const Variant* variants_k3s2(int* n);
 const Variant* variants_k1(int* n);
+const Variant* variants_point(int* n);
 
 // Generic fallback: one thread per output, FP32 fused multiply-add in
 // (ic, ky, kx) order. Used only for shapes without an MFMA variant.
@@ -130,7 +132,7 @@ const std::vector<Variant>& variants()
 {
     static const std::vector<Variant> table = [] {
         std::vector<Variant> t{Variant{"direct_fp32", 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr}};
-        for (auto family : {variants_k3s1, variants_k3s2, variants_k1}) {
+        for (auto family : {variants_k3s1, variants_k3s2, variants_k1, variants_point}) {
             int n = 0;
             const Variant* v = family(&n);
             t.insert(t.end(), v, v + n);
@@ -255,7 +257,50 @@ bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
     if (k.ws_ic && (static_cast<std::uint64_t>(d.ic) + k.kc) * static_cast<std::uint64_t>(ih) * iw * 2 >= (1ull << 31))
         return false;
     const bool flat = ih == 1 && oh == 1 && d.kh == 1 && d.kw == 1;
+    // conv_point_kernel: whole passes of channels, pixel rows on 4 bytes, a
+    // concat split on a 16-channel step, offsets below 2^31; no ReGLU. Its
+    // split form: split convs of a plain input and up to eight splits (a wave
+    // each).
+    if (k.point_ic && (!flat || !flat_1x1(d) || d.ic % k.point_ic != 0 || iw % 2 != 0 || d.ic_split % 16 != 0 ||
+                       (d.ksplit > 1) != k.point_split || (k.point_split && (concat(d) || d.ksplit > 8)) || d.epilogue == MLVC_EPI_REGLU || static_cast<std::uint64_t>(d.ic) * iw * 2 >= (1ull << 31) ||
+                       static_cast<std::uint64_t>((d.oc + k.bm - 1) / k.bm) * k.bm * d.ic * 2 >= (1ull << 31)))
+        return false;
     return !(d.kh == 1 && flat != (k.th == 1));
+}
+
+// Estimated time of a launch, to rank the variants of a geometry.
+//
+// Measured variants (us): a launch of W workgroups of K 16-channel steps each
+// takes
+//   cost[0] + cost[1] * K + w * (cost[2] + cost[3] * K),  w = max(1, W / CUs):
+// the launch and the first workgroup's latency chain, then each CU's share of
+// the work. The four numbers of each variant are a non-negative least-squares
+// fit (relative error) to its times over random geometries of its kernel size
+// (conv_point.hip, conv_k1.hip), three inputs in turn. On 400 1x1 convs the
+// pick is 2.4% off the fastest variant on the geometric mean (at most 40%);
+// counting rounds of two workgroups per CU, as below, it was 38% off.
+// The other variants: rounds of two workgroups per CU, work per round in MACs
+// plus a fixed overhead per tile.
+double plan_cost(const mlvc_hip_conv_desc& d, const Variant& k)
+{
+    int ih, iw, oh, ow;
+    kernel_geometry(d, ih, iw, oh, ow);
+    const long long tiles = static_cast<long long>((oh + k.th - 1) / k.th) * ((ow + k.tw - 1) / k.tw) *
+                            ((d.oc + k.bm - 1) / k.bm) * d.n;
+    if (k.cost[0] > 0.0f) {
+        const int splits = std::max(d.ksplit, 1);  // in one workgroup or in one each
+        const double steps = (d.ic + 15) / 16, wgs = static_cast<double>(tiles) * (k.point_split ? 1 : splits);
+        const double w = std::max(1.0, wgs / cu_count()), kk = std::ceil(steps / splits);
+        return k.cost[0] + k.cost[1] * kk + w * (k.cost[2] + k.cost[3] * kk);
+    }
+    const long long slots = 2 * cu_count(), rounds = (tiles + slots - 1) / slots;
+    double cost = static_cast<double>(rounds) * (static_cast<double>(k.bm) * k.th * k.tw + 4096.0);
+    // Ragged rows without the ragged builds are staged pixel by pixel, 16 or
+    // 32 two-byte loads each: 3 to 12 times the time of the row staging over
+    // 3x3 convs of 27 to 369 pixels wide (256->256 stride 2 on 58x103: 213 us
+    // against 18 us; 64->64 on 127x226: 27 against 9).
+    if (row_staged(d) && !k.launch_rag[0] && (iw % 8 != 0 || (k.ws_ic && ow % 8 != 0))) cost *= 8.0;
+    return cost;
 }
 
 }  // namespace
@@ -271,24 +316,11 @@ int mlvc_hip_conv_plan(mlvc_hip_conv_desc* desc)
         validate(*desc, false);
         split_rule(*desc, desc->ksplit, desc->split_c);
         const mlvc_hip_conv_desc& d = *desc;
-        int ih, iw, oh, ow;
-        kernel_geometry(d, ih, iw, oh, ow);
-        const int slots = 2 * cu_count();
         int best = 0;
         double best_cost = 0.0;
         for (int v = 1; v < variant_count(); ++v) {
             if (!eligible(d, variants()[v])) continue;
-            const Variant& k = variants()[v];
-            const long tiles = static_cast<long>((oh + k.th - 1) / k.th) * ((ow + k.tw - 1) / k.tw) *
-                               ((d.oc + k.bm - 1) / k.bm) * d.n;
-            const long rounds = (tiles + slots - 1) / slots;
-            // Work per round in MACs plus a fixed per-tile overhead.
-            double cost = static_cast<double>(rounds) * (static_cast<double>(k.bm) * k.th * k.tw + 4096.0);
-            // Ragged rows without the ragged builds are staged pixel by pixel,
-            // 16 or 32 two-byte loads each: 3 to 12 times the time of the row
-            // staging over 3x3 convs of 27 to 369 pixels wide (256->256 stride 2
-            // on 58x103: 213 us against 18 us; 64->64 on 127x226: 27 against 9).
-            if (row_staged(d) && !k.launch_rag[0] && (iw % 8 != 0 || (k.ws_ic && ow % 8 != 0))) cost *= 8.0;
+            const double cost = plan_cost(d, variants()[v]);
             if (best == 0 || cost < best_cost) {
                 best = v;
                 best_cost = cost;
@@ -357,23 +389,23 @@ int mlvc_hip_conv_pack(const mlvc_hip_conv_desc* desc, const uint16_t* w, void* 
             return;
         }
         const int taps = k.kh * k.kw, ks_n = k.kc / 16, mt_n = k.bm / 32;
-        const int ocb_n = (d.oc + k.bm - 1) / k.bm, chunks = (d.ic + k.kc - 1) / k.kc;
-        size_t o = 0;
+        const int chunks = (d.ic + k.kc - 1) / k.kc;
         // Layout [ocb][chunk][tap][ks][mt][lane][8]: lane l of m-tile mt
         // holds W[oc = ocb*BM + mt*32 + l%32][ic = chunk*KC + ks*16 + 8*(l/32) + j][tap].
-        for (int ocb = 0; ocb < ocb_n; ++ocb)
-            for (int ch = 0; ch < chunks; ++ch)
-                for (int tap = 0; tap < taps; ++tap)
-                    for (int ks = 0; ks < ks_n; ++ks)
-                        for (int mt = 0; mt < mt_n; ++mt)
-                            for (int lane = 0; lane < 64; ++lane)
-                                for (int j = 0; j < 8; ++j) {
-                                    const int oc = ocb * k.bm + mt * 32 + (lane & 31);
-                                    const int ic = ch * k.kc + ks * 16 + 8 * (lane >> 5) + j;
-                                    out[o++] = (oc < d.oc && ic < d.ic)
-                                                   ? w[(static_cast<size_t>(oc) * d.ic + ic) * taps + tap]
-                                                   : std::uint16_t{0};
-                                }
+        // Written in source order: 8 channels of one row are read as they
+        // lie, a lane's 16 bytes are written per tap.
+        if (d.oc % k.bm != 0 || d.ic % k.kc != 0) std::memset(out, 0, mlvc_hip_conv_packed_bytes(desc));
+        const size_t tap_stride = static_cast<size_t>(ks_n) * mt_n * 512;
+        for (int oc = 0; oc < d.oc; ++oc)
+            for (int ic = 0; ic < d.ic; ic += 8) {
+                const int ocb = oc / k.bm, mt = oc % k.bm / 32, ch = ic / k.kc, ks = ic % k.kc / 16;
+                const int lane = oc % 32 + 32 * (ic % 16 / 8), n = std::min(8, d.ic - ic);
+                std::uint16_t* o = out + (static_cast<size_t>(ocb) * chunks + ch) * taps * tap_stride +
+                                   (static_cast<size_t>(ks) * mt_n + mt) * 512 + lane * 8;
+                const std::uint16_t* src = w + (static_cast<size_t>(oc) * d.ic + ic) * taps;
+                for (int tap = 0; tap < taps; ++tap, o += tap_stride)
+                    for (int j = 0; j < n; ++j) o[j] = src[j * taps + tap];
+            }
     });
 }
 
@@ -453,7 +485,11 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             const std::uint64_t plane = static_cast<std::uint64_t>(a.ih) * a.iw;
             const bool images4 = d.n == 1 || ((a.x2 ? a.ic_split : d.ic) * plane % 2 == 0 &&
                                               (!a.x2 || (d.ic - a.ic_split) * plane % 2 == 0));
-            const bool vec = rows && even;
+            if (k.point_ic && (a.ih != 1 || d.ic % k.point_ic != 0 || a.iw % 2 != 0 || a.s2d > 1 || a.d2s > 1 ||
+                               (a.ksplit > 1) != k.point_split || (k.point_split && (d.x2 || a.ksplit > 8)) ||
+                               (d.x2 && d.ic_split % 16 != 0) || d.epilogue == MLVC_EPI_REGLU))
+                throw std::runtime_error("conv: variant does not match the geometry");
+            const bool vec = rows && (even || k.point_ic);
             const auto ragged = rows && !even && images4 ? k.launch_rag[a.iw & 1] : nullptr;
             a.tiles_x = (a.ow + k.tw - 1) / k.tw;
             a.nchunks = (d.ic + k.kc - 1) / k.kc;
@@ -471,7 +507,7 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             if (k.ws_ic && (d.x2 || a.s2d > 1)) throw std::runtime_error("conv: variant needs a plain input");
             if (k.ws_ic && !vec && (even || !k.launch_scalar)) throw std::runtime_error("conv: variant needs 16-byte row staging");
             (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : ragged ? ragged : k.launch_scalar)(a, grid, to_stream(s));
-            if (a.ksplit > 1) {
+            if (a.ksplit > 1 && !(k.point_split && vec)) {
                 ConvArgs r = a;  // the reduce works in the real output geometry
                 r.ih = d.ih;
                 r.iw = d.iw;

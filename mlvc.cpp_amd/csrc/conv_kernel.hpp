@@ -822,6 +822,13 @@ struct Variant {
     // Its channel-last output tile fits the LDS: bit 0 plain, bit 1 with
     // DEPTH_TO_SPACE(2).
     int nhwc_out = 0;
+    // conv_point_kernel (conv_point.hpp): the input channels must be a
+    // multiple of point_ic; 0 for the other kernels.
+    int point_ic = 0;
+    // conv_point_split_kernel: split convs only, all splits in one workgroup.
+    bool point_split = false;
+    // Measured cost (see plan_cost in conv_igemm.hip), or all zero.
+    float cost[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     // Row staging of widths that are no multiple of 8: even, odd (or null:
     // such widths are staged pixel by pixel, by launch_scalar).
     void (*launch_rag[2])(const ConvArgs&, dim3, hipStream_t) = {nullptr, nullptr};
@@ -831,6 +838,15 @@ template <class C>
 void launch_mfma(const ConvArgs& a, dim3 grid, hipStream_t s)
 {
     hipLaunchKernelGGL(conv_mfma_kernel<C>, grid, dim3(C::kThreads), 0, s, a);
+}
+
+constexpr Variant costed(Variant v, float launch, float step, float group, float group_step)
+{
+    v.cost[0] = launch;
+    v.cost[1] = step;
+    v.cost[2] = group;
+    v.cost[3] = group_step;
+    return v;
 }
 
 // A one-stage variant with row staging of ragged widths (STG 3 and 4).
