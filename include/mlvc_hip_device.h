@@ -50,6 +50,7 @@ int mlvc_hip_event_create(mlvc_hip_event* e);
 int mlvc_hip_event_destroy(mlvc_hip_event e);
 int mlvc_hip_event_record(mlvc_hip_event e, mlvc_hip_stream s);
 int mlvc_hip_event_synchronize(mlvc_hip_event e);
+int mlvc_hip_stream_wait_event(mlvc_hip_stream s, mlvc_hip_event e); /* work queued later on s waits for e */
 int mlvc_hip_event_elapsed_ms(mlvc_hip_event start, mlvc_hip_event stop, float* ms);
 
 /* ---- hipGraph capture/replay (driver.cpp:452-489 begin_capture/
@@ -258,6 +259,12 @@ int mlvc_hip_space_to_depth(const void* x, void* y, int n, int in_c, int h, int 
 
 /* ---- elementwise (elementwise.cu:1-80): y = fp16(op(fp32 inputs)) ---- */
 int mlvc_hip_leaky_relu(const void* x, void* y, size_t count, float alpha, mlvc_hip_stream s);
+
+/* Device -> pinned host memory by a copy kernel of a few workgroups, for
+ * downloads that run under other kernels. Both pointers 16-byte aligned. */
+int mlvc_hip_download(const void* src, void* dst_host, size_t bytes, mlvc_hip_stream s);
+/* *dst = value (a kernel argument, so nothing on the host is read later). */
+int mlvc_hip_store_i32(int32_t* dst, int32_t value, mlvc_hip_stream s);
 
 /* ---- Codec I/O around the encoder / decoder graphs ----
  * Frames are I420 bytes (Y w*h, then U and V (w/2)*(h/2)); the model image

@@ -200,13 +200,18 @@ public:
         // Pending codec slots and any queued work finish before buffers go.
         mlvc_hip_set_device(device_);
         mlvc_hip_stream_synchronize(stream_);
+        for (auto st : {up_, down_})
+            if (st) mlvc_hip_stream_synchronize(st);
         for (auto& sl : slots_)
-            if (sl.done) mlvc_hip_event_destroy(sl.done);
+            for (auto e : {sl.uploaded, sl.computed, sl.done})
+                if (e) mlvc_hip_event_destroy(e);
         for (auto g : graphs_) mlvc_hip_graph_destroy(g);
         mlvc_hip_event_destroy(ev0_);
         mlvc_hip_event_destroy(ev1_);
         for (auto e : frame_evs_) mlvc_hip_event_destroy(e);
         if (flush_buf_) mlvc_hip_free(flush_buf_);
+        for (auto st : {up_, down_})
+            if (st) mlvc_hip_stream_destroy(st);
         mlvc_hip_stream_destroy(stream_);
     }
 
@@ -230,9 +235,20 @@ public:
     // (backends/driver_cubin/src/cuda_graph_executor.cpp:156-400) with the
     // checks of the CPU backend's configure_codec_io
     // (backends/cpu/src/execution_plan.cpp:1386-1486): per slot a pinned
-    // frame, pinned copies of the graph's external outputs (encoder) or
-    // inputs (decoder) and an event; submits run upload -> conversion kernel
-    // -> frame graph -> download on the backend's stream.
+    // frame and pinned copies of the graph's external outputs (encoder) or
+    // inputs (decoder), with a device copy of each, and three events.
+    // Submits run upload -> conversion kernel -> frame graph -> download, the
+    // graphs in submit order on the backend's stream. A 1080p frame's 3.1 MB
+    // and its latent's 4.2 MB take 63 and 83 us on the link, a quarter of its
+    // graph's time, so a submit among others (pipelined()) takes them on a
+    // stream each way, under the other frames' graphs: through device
+    // copies that are the slot's own (nothing overwrites them before the slot
+    // is waited for), since the next graph writes over the encoder's outputs
+    // and the decoder's inputs are in use by the one before. The device copy
+    // is about 4 us. Four 1080p frames in flight: encoder 2637 -> 2330 us,
+    // decoder 1711 -> 1385 us. A submit on its own has nothing to run under, and
+    // the hops between streams and the slower download cost 30 us of 657: it
+    // is one chain on the backend's stream.
     void configure_codec_io(const CodecIoConfig& cfg)
     {
         if (codec_on_) fail("codec I/O is already configured");
@@ -277,7 +293,8 @@ public:
         if (q < 0 || img < 0) fail("missing required codec I/O tensors");
 
         select();
-        codec_frame_ = DeviceMem(frame_bytes);
+        for (auto* st : {&up_, &down_})
+            if (!*st) hip_check(mlvc_hip_stream_create(st), "stream creation");
         if (encoder) {
             std::uint16_t lut[256];
             for (int v = 0; v < 256; ++v) lut[v] = float_to_half((static_cast<float>(v) / 255.0F) * cfg.pixel_range);
@@ -289,16 +306,19 @@ public:
         for (CodecSlot& sl : slots) {
             sl.frame = HostMem(frame_bytes);
             std::memset(sl.frame.ptr, 0, frame_bytes);
-            sl.q = HostMem(sizeof(std::int32_t));
+            sl.frame_dev = DeviceMem(frame_bytes);
             const auto& ids = encoder ? ext_out_ : ext_in_;
             sl.io.resize(ids.size());
+            sl.io_dev.resize(ids.size());
             for (std::size_t i = 0; i < ids.size(); ++i)
                 if (encoder || static_cast<int>(i) != q) {
                     sl.io[i] = HostMem(desc_bytes(desc(ids[i])));
                     std::memset(sl.io[i].ptr, 0, desc_bytes(desc(ids[i])));
+                    sl.io_dev[i] = DeviceMem(desc_bytes(desc(ids[i])));
                 }
-            hip_check(mlvc_hip_event_create(&sl.done), "event creation");
         }
+        for (CodecSlot& sl : slots)
+            for (auto* e : {&sl.uploaded, &sl.computed, &sl.done}) hip_check(mlvc_hip_event_create(e), "event creation");
         slots_ = std::move(slots);
         codec_ = cfg;
         codec_frame_bytes_ = frame_bytes;
@@ -323,20 +343,29 @@ public:
         const std::int32_t q32 = static_cast<std::int32_t>(shifted_q);
         check_gather_indices(static_cast<std::size_t>(codec_q_), &q32);
         select();
-        hip_check(mlvc_hip_memcpy_h2d(codec_frame_.ptr, sl.frame.ptr, codec_frame_bytes_, stream_), "frame upload");
+        const bool overlap = pipelined();
+        hip_check(mlvc_hip_memcpy_h2d(sl.frame_dev.ptr, sl.frame.ptr, codec_frame_bytes_, overlap ? up_ : stream_), "frame upload");
+        if (overlap) uploaded(sl);
         const FramePadding& pad = codec_.padding;
-        hip_check(mlvc_hip_yuv420_to_model(static_cast<const std::uint8_t*>(codec_frame_.ptr),
+        hip_check(mlvc_hip_yuv420_to_model(static_cast<const std::uint8_t*>(sl.frame_dev.ptr),
                                            static_cast<const std::uint16_t*>(codec_lut_.ptr),
                                            input_buf_.at(ext_in_[static_cast<std::size_t>(codec_img_)]).ptr, codec_.width,
                                            codec_.height, codec_.model_width, codec_.model_height, pad.rotated ? 1 : 0,
                                            stream_),
                   "frame conversion");
-        enqueue_q(sl, shifted_q);
+        enqueue_q(shifted_q);
         hip_check(mlvc_hip_graph_launch(graphs_[static_cast<std::size_t>(parity_)], stream_), "graph launch");
-        for (std::size_t i = 0; i < ext_out_.size(); ++i)
-            hip_check(mlvc_hip_memcpy_d2h(sl.io[i].ptr, ptr(ext_out_[i], parity_), desc_bytes(desc(ext_out_[i])), stream_),
+        if (overlap) {
+            for (std::size_t i = 0; i < ext_out_.size(); ++i) device_copy(sl.io_dev[i].ptr, ptr(ext_out_[i], parity_), ext_out_[i]);
+            computed(sl);
+        }
+        for (std::size_t i = 0; i < ext_out_.size(); ++i) {
+            const std::size_t bytes = desc_bytes(desc(ext_out_[i]));
+            hip_check(overlap ? mlvc_hip_download(sl.io_dev[i].ptr, sl.io[i].ptr, bytes, down_)
+                              : mlvc_hip_memcpy_d2h(sl.io[i].ptr, ptr(ext_out_[i], parity_), bytes, stream_),
                       "output download");
-        finish_submit(sl);
+        }
+        finish_submit(sl, overlap ? down_ : stream_);
     }
 
     std::vector<TensorView> encoder_outputs(std::size_t index) const
@@ -369,21 +398,31 @@ public:
         const std::int32_t q32 = static_cast<std::int32_t>(shifted_q);
         check_gather_indices(static_cast<std::size_t>(codec_q_), &q32);
         select();
+        const bool overlap = pipelined();
         for (std::size_t i = 0; i < ext_in_.size(); ++i) {
             if (static_cast<int>(i) == codec_q_) continue;
-            hip_check(mlvc_hip_memcpy_h2d(input_buf_.at(ext_in_[i]).ptr, sl.io[i].ptr, desc_bytes(desc(ext_in_[i])), stream_),
+            hip_check(mlvc_hip_memcpy_h2d(overlap ? sl.io_dev[i].ptr : input_buf_.at(ext_in_[i]).ptr, sl.io[i].ptr,
+                                          desc_bytes(desc(ext_in_[i])), overlap ? up_ : stream_),
                       "input upload");
         }
-        enqueue_q(sl, shifted_q);
+        if (overlap) {
+            uploaded(sl);
+            for (std::size_t i = 0; i < ext_in_.size(); ++i)
+                if (static_cast<int>(i) != codec_q_) device_copy(input_buf_.at(ext_in_[i]).ptr, sl.io_dev[i].ptr, ext_in_[i]);
+        }
+        enqueue_q(shifted_q);
         hip_check(mlvc_hip_graph_launch(graphs_[static_cast<std::size_t>(parity_)], stream_), "graph launch");
         const FramePadding& pad = codec_.padding;
         hip_check(mlvc_hip_model_to_yuv420(ptr(ext_out_[static_cast<std::size_t>(codec_img_)], parity_),
-                                           static_cast<std::uint8_t*>(codec_frame_.ptr), codec_.width, codec_.height,
+                                           static_cast<std::uint8_t*>(sl.frame_dev.ptr), codec_.width, codec_.height,
                                            codec_.model_width, codec_.model_height, pad.left, pad.top,
                                            pad.rotated ? 1 : 0, codec_.pixel_range, stream_),
                   "frame conversion");
-        hip_check(mlvc_hip_memcpy_d2h(sl.frame.ptr, codec_frame_.ptr, codec_frame_bytes_, stream_), "frame download");
-        finish_submit(sl);
+        if (overlap) computed(sl);
+        hip_check(overlap ? mlvc_hip_download(sl.frame_dev.ptr, sl.frame.ptr, codec_frame_bytes_, down_)
+                          : mlvc_hip_memcpy_d2h(sl.frame.ptr, sl.frame_dev.ptr, codec_frame_bytes_, stream_),
+                  "frame download");
+        finish_submit(sl, overlap ? down_ : stream_);
     }
 
     Yuv420FrameView decoder_output_yuv(std::size_t index) const
@@ -2273,8 +2312,9 @@ private:
     struct CodecSlot {
         HostMem frame;            // encoder input / decoder output frame (I420)
         std::vector<HostMem> io;  // encoder: external outputs; decoder: external inputs (not q)
-        HostMem q;                // q_index_shifted staging
-        mlvc_hip_event done = nullptr;
+        DeviceMem frame_dev;      // device copies of frame and io
+        std::vector<DeviceMem> io_dev;
+        mlvc_hip_event uploaded = nullptr, computed = nullptr, done = nullptr;
         bool pending = false;
     };
 
@@ -2307,18 +2347,52 @@ private:
 
     Yuv420FrameView frame_view(const CodecSlot& sl) const { return frame_view(const_cast<CodecSlot&>(sl)); }
 
-    void enqueue_q(CodecSlot& sl, int shifted_q)
+    // q is a kernel argument: a copy of 4 bytes between two kernels waits
+    // behind every download in flight.
+    void enqueue_q(int shifted_q)
     {
-        const std::int32_t q32 = static_cast<std::int32_t>(shifted_q);
-        std::memcpy(sl.q.ptr, &q32, sizeof(q32));
-        hip_check(mlvc_hip_memcpy_h2d(input_buf_.at(ext_in_[static_cast<std::size_t>(codec_q_)]).ptr, sl.q.ptr, sizeof(q32), stream_),
-                  "q upload");
+        hip_check(mlvc_hip_store_i32(static_cast<std::int32_t*>(input_buf_.at(ext_in_[static_cast<std::size_t>(codec_q_)]).ptr),
+                                     static_cast<std::int32_t>(shifted_q), stream_),
+                  "q store");
     }
 
-    void finish_submit(CodecSlot& sl)
+    // The backend's stream goes on when the slot's uploads are in; the
+    // download stream when the slot's results are.
+    void uploaded(CodecSlot& sl)
+    {
+        hip_check(mlvc_hip_event_record(sl.uploaded, up_), "event record");
+        hip_check(mlvc_hip_stream_wait_event(stream_, sl.uploaded), "stream wait");
+    }
+
+    void computed(CodecSlot& sl)
+    {
+        hip_check(mlvc_hip_event_record(sl.computed, stream_), "event record");
+        hip_check(mlvc_hip_stream_wait_event(down_, sl.computed), "stream wait");
+    }
+
+    // A whole FP16 or INT32 tensor (buffers are 256-byte aligned, and so
+    // are arena offsets), on the backend's stream.
+    void device_copy(void* dst, const void* src, TensorId id)
+    {
+        const std::size_t halves = desc_bytes(desc(id)) / 2;
+        hip_check(mlvc_hip_copy_rows(src, dst, 1, halves, halves, halves, stream_), "device copy");
+    }
+
+    // Whether this submit's transfers may have other frames' graphs to run
+    // under: other slots are in flight, or were at the previous submit (the
+    // first of a burst after the last one was waited for).
+    bool pipelined()
+    {
+        const bool others = std::any_of(slots_.begin(), slots_.end(), [](const CodecSlot& sl) { return sl.pending; });
+        const bool before = codec_piped_;
+        codec_piped_ = others;
+        return others || before;
+    }
+
+    void finish_submit(CodecSlot& sl, mlvc_hip_stream last)
     {
         advance();
-        hip_check(mlvc_hip_event_record(sl.done, stream_), "event record");
+        hip_check(mlvc_hip_event_record(sl.done, last), "event record");
         sl.pending = true;
     }
 
@@ -2326,6 +2400,7 @@ private:
     std::string model_;
     aot::LoadedGraph graph_;
     mlvc_hip_stream stream_ = nullptr;
+    mlvc_hip_stream up_ = nullptr, down_ = nullptr;  // codec slots' transfers
     mlvc_hip_event ev0_ = nullptr, ev1_ = nullptr;
     void ensure_flush_buffer(std::size_t flush_bytes)
     {
@@ -2361,11 +2436,12 @@ private:
     int parity_ = 0;
     bool initialized_ = false;
     // codec I/O
+    bool codec_piped_ = false;
     bool codec_on_ = false, codec_encoder_ = false;
     CodecIoConfig codec_{};
     std::size_t codec_frame_bytes_ = 0;
     int codec_q_ = -1, codec_img_ = -1;  // external input index of q; of x (encoder) / output index of x_hat (decoder)
-    DeviceMem codec_frame_, codec_lut_;
+    DeviceMem codec_lut_;
     std::vector<CodecSlot> slots_;
 };
 

@@ -115,6 +115,11 @@ int mlvc_hip_event_synchronize(mlvc_hip_event e)
     return guard([&] { check(hipEventSynchronize(reinterpret_cast<hipEvent_t>(e)), "hipEventSynchronize"); });
 }
 
+int mlvc_hip_stream_wait_event(mlvc_hip_stream s, mlvc_hip_event e)
+{
+    return guard([&] { check(hipStreamWaitEvent(to_stream(s), reinterpret_cast<hipEvent_t>(e), 0), "hipStreamWaitEvent"); });
+}
+
 int mlvc_hip_event_elapsed_ms(mlvc_hip_event start, mlvc_hip_event stop, float* ms)
 {
     return guard([&] {

@@ -260,3 +260,68 @@ def test_run_takes_int32_control_input(pair):
     x_hat = dec.run([y, np.array([2], np.int32)])[0]
     assert x_hat.shape == (1, 3, MH, MW)
     dec.close()
+
+
+# Submits that find other slots in flight transfer on their own streams
+# through the slot's device copies; a lone submit is one chain. Any mix of the
+# two must give what frames submitted and waited for one by one give.
+@pytest.mark.parametrize("bursts", [(1, 3, 1, 4, 2), (4, 4, 1)])
+def test_bursts_equal_single_submits(pair, bursts):
+    d, bindings = pair
+    w, h, slots, total = 128, 60, 4, sum(bursts)
+    rng = np.random.default_rng(33)
+    clips = [rng.integers(0, 256, O.yuv_frame_bytes(w, h), dtype=np.uint8) for _ in range(total)]
+
+    def encode(pattern):
+        enc = backend(d, "MLVCEncoder", bindings)
+        enc.configure_codec_io(w, h, MW, MH, padding=O.frame_padding(w, h, MW, MH), slots=slots)
+        enc.reset_state()
+        out, k = [], 0
+        for n in pattern:
+            for s in range(n):
+                enc.encoder_input_yuv(s)[:] = clips[k + s]
+                enc.submit_encoder(s, k + s)
+            for s in reversed(range(n)):  # waited for in another order than submitted
+                enc.wait_codec_slot(s)
+            out += [[np.array(o) for o in enc.encoder_outputs(s)] for s in range(n)]
+            k += n
+        enc.close()
+        return out
+
+    def decode(pattern, latents):
+        dec = backend(d, "MLVCDecoder", bindings)
+        dec.configure_codec_io(w, h, MW, MH, padding=O.frame_padding(w, h, MW, MH), slots=slots)
+        dec.reset_state()
+        out, k = [], 0
+        for n in pattern:
+            for s in range(n):
+                for dst, src in zip(dec.decoder_inputs(s), latents[k + s]):
+                    dst.reshape(-1)[:] = src.reshape(-1)
+                dec.submit_decoder(s, k + s)
+            for s in range(n):
+                dec.wait_codec_slot(s)
+            out += [np.array(dec.decoder_output_yuv(s)) for s in range(n)]
+            k += n
+        dec.close()
+        return out
+
+    ones = (1,) * total
+    want, got = encode(ones), encode(bursts)
+    for i, (a, b) in enumerate(zip(want, got)):
+        assert all(np.array_equal(x, y) for x, y in zip(a, b)), f"encoded frame {i}"
+    for i, (a, b) in enumerate(zip(decode(ones, want), decode(bursts, want))):
+        assert np.array_equal(a, b), f"decoded frame {i}"
+
+
+@pytest.mark.parametrize("count", [1, 15, 16, 17, 4096, 16 * 256 * 4 + 16, 99991])
+def test_download_copies_every_byte(dev, count):
+    rng = np.random.default_rng(count)
+    data = rng.integers(0, 256, count, dtype=np.uint8)
+    src, out = dev.put(data), C.c_void_p()
+    dev.check(dev.lib.mlvc_hip_host_alloc(C.byref(out), C.c_size_t(count + 16)))
+    host = np.ctypeslib.as_array(C.cast(out, C.POINTER(C.c_uint8)), (count + 16,))
+    host[:] = 7
+    dev.check(dev.lib.mlvc_hip_download(src, out, C.c_size_t(count), None))
+    dev.check(dev.lib.mlvc_hip_stream_synchronize(None))
+    assert np.array_equal(host[:count], data) and (host[count:] == 7).all()
+    dev.check(dev.lib.mlvc_hip_host_free(out))
