@@ -249,6 +249,7 @@ bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
     // no ReGLU, DEPTH_TO_SPACE(2) or none; rows of a multiple of 8 pixels in
     // and out, or of any width where the variant has ragged builds (NCHW).
     if (k.ws_ic && (concat(d) || d.in_s2d_block > 1 || d.epilogue == MLVC_EPI_REGLU || d.out_d2s_block > 2)) return false;
+    if (k.ws_ic && k.ws_mult > 16 && d.ic % k.ws_mult != 0) return false;
     if (k.ws_ic && (d.iw % 8 != 0 || d.ow % 8 != 0) && (!k.launch_rag[0] || d.in_nhwc || d.out_nhwc)) return false;
     int ih, iw, oh, ow;
     kernel_geometry(d, ih, iw, oh, ow);
@@ -272,35 +273,60 @@ bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
 //
 // Measured variants (us): a launch of W workgroups of K 16-channel steps each
 // takes
-//   cost[0] + cost[1] * K + w * (cost[2] + cost[3] * K),  w = max(1, W / CUs):
-// the launch and the first workgroup's latency chain, then each CU's share of
-// the work. The four numbers of each variant are a non-negative least-squares
-// fit (relative error) to its times over random geometries of its kernel size
-// (conv_point.hip, conv_k1.hip), three inputs in turn. On 400 1x1 convs the
-// pick is 2.4% off the fastest variant on the geometric mean (at most 40%);
-// counting rounds of two workgroups per CU, as below, it was 38% off.
-// The other variants: rounds of two workgroups per CU, work per round in MACs
-// plus a fixed overhead per tile.
-double plan_cost(const mlvc_hip_conv_desc& d, const Variant& k)
+//   cost[0] + cost[1] * K + w * (cost[2] + cost[3] * K):
+// the launch and the first workgroup's latency chain, then each CU's share w
+// of the work: max(1, W / CUs) for the short 1x1 workgroups, whole workgroups
+// per CU, ceil(W / CUs), for the long 3x3 ones. The four numbers of each
+// variant are a non-negative least-squares fit (relative error) to its times
+// over random geometries of its kernel size, three inputs in turn (3x3: then
+// scaled by up to 15% where that improves the picks). The pick's distance from
+// the fastest variant, geometric mean (and by rounds of two workgroups per
+// CU, as below): 400 1x1 convs 2.4% (38%), 189 3x3 stride-1 convs 2.3% (24%),
+// 69 stride-2 ones 1.5% (19%); on 160 convs outside the fit 2.5, 2.0 and 4.2%.
+double measured_cost(const mlvc_hip_conv_desc& d, const Variant& k, int ow, long long tiles)
 {
-    int ih, iw, oh, ow;
-    kernel_geometry(d, ih, iw, oh, ow);
-    const long long tiles = static_cast<long long>((oh + k.th - 1) / k.th) * ((ow + k.tw - 1) / k.tw) *
-                            ((d.oc + k.bm - 1) / k.bm) * d.n;
-    if (k.cost[0] > 0.0f) {
-        const int splits = std::max(d.ksplit, 1);  // in one workgroup or in one each
-        const double steps = (d.ic + 15) / 16, wgs = static_cast<double>(tiles) * (k.point_split ? 1 : splits);
-        const double w = std::max(1.0, wgs / cu_count()), kk = std::ceil(steps / splits);
-        return k.cost[0] + k.cost[1] * kk + w * (k.cost[2] + k.cost[3] * kk);
-    }
+    const int splits = std::max(d.ksplit, 1);  // in one workgroup or in one each
+    const double steps = (d.ic + 15) / 16, kk = std::ceil(steps / splits);
+    const double share = static_cast<double>(tiles) * (k.point_split ? 1 : splits) / cu_count();
+    const double w = k.kh == 1 ? std::max(1.0, share) : std::ceil(share);
+    const double cost = k.cost[0] + k.cost[1] * kk + w * (k.cost[2] + k.cost[3] * kk);
+    // 3x3 rows that are no multiple of 8: without ragged builds they are
+    // staged pixel by pixel, 16 or 32 two-byte loads each, 3 to 12 times the
+    // time of the row staging (256->256 stride 2 on 58x103: 213 against 18 us;
+    // 64->64 on 127x226: 27 against 9). conv_mfma_kernel's ragged builds
+    // stage every 16 channels anew and run up to 1.5 times their estimate.
+    if (k.kh == 1 || (d.iw % 8 == 0 && (!k.ws_ic || ow % 8 == 0))) return cost;
+    return cost * (!k.launch_rag[0] ? 8.0 : k.ws_ic ? 1.0 : 1.5);
+}
+
+// The other variants, and the geometries the measurements do not cover
+// (SPACE_TO_DEPTH inputs, 3x3 convs of a concat): rounds of two workgroups per
+// CU, work per round in MACs plus a fixed overhead per tile.
+double round_cost(const mlvc_hip_conv_desc& d, const Variant& k, int iw, int ow, long long tiles)
+{
     const long long slots = 2 * cu_count(), rounds = (tiles + slots - 1) / slots;
-    double cost = static_cast<double>(rounds) * (static_cast<double>(k.bm) * k.th * k.tw + 4096.0);
-    // Ragged rows without the ragged builds are staged pixel by pixel, 16 or
-    // 32 two-byte loads each: 3 to 12 times the time of the row staging over
-    // 3x3 convs of 27 to 369 pixels wide (256->256 stride 2 on 58x103: 213 us
-    // against 18 us; 64->64 on 127x226: 27 against 9).
-    if (row_staged(d) && !k.launch_rag[0] && (iw % 8 != 0 || (k.ws_ic && ow % 8 != 0))) cost *= 8.0;
-    return cost;
+    const double cost = static_cast<double>(rounds) * (static_cast<double>(k.bm) * k.th * k.tw + 4096.0);
+    return row_staged(d) && !k.launch_rag[0] && (iw % 8 != 0 || (k.ws_ic && ow % 8 != 0)) ? cost * 8.0 : cost;
+}
+
+// The variant of least cost; 0 (the direct fallback) where none is eligible.
+int best_variant(const mlvc_hip_conv_desc& d, bool measured)
+{
+    int ih, iw, oh, ow, best = 0;
+    kernel_geometry(d, ih, iw, oh, ow);
+    double best_cost = 0.0;
+    for (int v = 1; v < variant_count(); ++v) {
+        const Variant& k = variants()[v];
+        if ((measured && k.cost[3] + k.cost[2] <= 0.0f) || !eligible(d, k)) continue;
+        const long long tiles = static_cast<long long>((oh + k.th - 1) / k.th) * ((ow + k.tw - 1) / k.tw) *
+                                ((d.oc + k.bm - 1) / k.bm) * d.n;
+        const double cost = measured ? measured_cost(d, k, ow, tiles) : round_cost(d, k, iw, ow, tiles);
+        if (best == 0 || cost < best_cost) {
+            best = v;
+            best_cost = cost;
+        }
+    }
+    return best;
 }
 
 }  // namespace
@@ -316,16 +342,8 @@ int mlvc_hip_conv_plan(mlvc_hip_conv_desc* desc)
         validate(*desc, false);
         split_rule(*desc, desc->ksplit, desc->split_c);
         const mlvc_hip_conv_desc& d = *desc;
-        int best = 0;
-        double best_cost = 0.0;
-        for (int v = 1; v < variant_count(); ++v) {
-            if (!eligible(d, variants()[v])) continue;
-            const double cost = plan_cost(d, variants()[v]);
-            if (best == 0 || cost < best_cost) {
-                best = v;
-                best_cost = cost;
-            }
-        }
+        int best = row_staged(d) && (d.kh == 1 || !concat(d)) ? best_variant(d, true) : 0;
+        if (best == 0) best = best_variant(d, false);
         desc->variant = best;
         if (best == 0) {  // the direct fallback sums every channel itself
             desc->ksplit = 1;
@@ -504,6 +522,8 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             const std::uint64_t src_plane = static_cast<std::uint64_t>(a.ih) * a.iw * 4 * 2;
             const bool s2d_vec = k.launch_s2d && a.s2d == 2 && (reinterpret_cast<std::uintptr_t>(d.x) & 15u) == 0 &&
                                  a.iw % 8 == 0 && (static_cast<std::uint64_t>(d.ic / 4) + k.kc / 4 + 1) * src_plane < (1ull << 31);
+            if (k.ws_ic && k.ws_mult > 16 && d.ic % k.ws_mult != 0)
+                throw std::runtime_error("conv: variant does not match the geometry");
             if (k.ws_ic && (d.x2 || a.s2d > 1)) throw std::runtime_error("conv: variant needs a plain input");
             if (k.ws_ic && !vec && (even || !k.launch_scalar)) throw std::runtime_error("conv: variant needs 16-byte row staging");
             (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : ragged ? ragged : k.launch_scalar)(a, grid, to_stream(s));

@@ -27,7 +27,7 @@ const Variant kTable[] = {
     MLVC_VARIANT_WS2(128, 2, 64, 32, 2, 4),
     MLVC_VARIANT_WS2(128, 2, 32, 64, 2, 4),
     MLVC_VARIANT_WS2(128, 4, 32, 64, 1, 4),
-    with_ragged_ws<WsCfg<128, 2, 32, 32, 2, 2, 4>>(MLVC_VARIANT_WS2(128, 2, 32, 32, 2, 4)),
+    MLVC_VARIANT_WS2(128, 2, 32, 32, 2, 4),
     MLVC_VARIANT_WS2(192, 4, 32, 32, 2, 3),
     MLVC_VARIANT_WS2(192, 2, 32, 64, 2, 3),
     // Deeper A rings, six waves over 192 output channels (one m-tile
@@ -36,8 +36,11 @@ const Variant kTable[] = {
     MLVC_VARIANT_WS2R(192, 2, 32, 64, 2, 6, 9),
     MLVC_VARIANT_WS2R(128, 4, 24, 32, 2, 4, 9),
     // Short, narrow tiles for deep convs onto few pixels (46x80 outputs).
-    with_ragged_ws<WsCfg<64, 2, 16, 64, 4, 2, 2, 9>>(MLVC_VARIANT_WS2R(64, 2, 16, 64, 4, 2, 9)),
-    with_ragged_ws<WsCfg<128, 2, 16, 64, 2, 2, 4, 9>>(MLVC_VARIANT_WS2R(128, 2, 16, 64, 2, 4, 9)),
+    costed(with_ragged_ws<WsCfg<64, 2, 16, 64, 4, 2, 2, 9>>(MLVC_VARIANT_WS2R(64, 2, 16, 64, 4, 2, 9)), 2.068f, 0.654f, 1.105f, 0.176f),
+    MLVC_VARIANT_WS2R(128, 2, 16, 64, 2, 4, 9),
+    // A ring of 18 fragments, as for stride 1.
+    costed(with_ragged_ws<WsCfg<64, 2, 16, 64, 2, 2, 2, 18>>(MLVC_VARIANT_WS2R(64, 2, 16, 64, 2, 2, 18)), 2.454f, 0.520f, 1.032f, 0.179f),
+    costed(with_ragged_ws<WsCfg<128, 2, 16, 64, 2, 2, 4, 18>>(MLVC_VARIANT_WS2R(128, 2, 16, 64, 2, 4, 18)), 2.358f, 0.316f, 1.551f, 0.308f),
     // All 192 output channels in one block over tiles dividing 136x240 (no
     // padded rows or columns), and one 32-pixel tile of all 256 channels per
     // CU at 68x120 (255 workgroups).
@@ -46,7 +49,7 @@ const Variant kTable[] = {
     MLVC_VARIANT_WS2R(256, 4, 8, 64, 2, 8, 9),
     // Four workgroups per CU (128 registers, 29 KB of LDS each): the
     // stride-2 convs wait on memory, and more waves keep more loads in flight.
-    with_ragged_ws<WsCfg<128, 2, 32, 32, 4, 2, 4>>(MLVC_VARIANT_WS2(128, 2, 32, 32, 4, 4)),
+    costed(with_ragged_ws<WsCfg<128, 2, 32, 32, 4, 2, 4>>(MLVC_VARIANT_WS2(128, 2, 32, 32, 4, 4)), 1.517f, 0.811f, 2.753f, 0.270f),
     // One 8x16 tile of all 192 output channels per CU at 136x240 (255
     // workgroups of six waves, 109 KB of LDS for two halo buffers): each CU
     // streams the 442 KB weight set of a 128 -> 192 conv once, where the

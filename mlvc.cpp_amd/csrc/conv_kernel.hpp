@@ -822,12 +822,14 @@ struct Variant {
     // Its channel-last output tile fits the LDS: bit 0 plain, bit 1 with
     // DEPTH_TO_SPACE(2).
     int nhwc_out = 0;
+    // ...and needs input channels in multiples of ws_mult.
+    int ws_mult = 1;
     // conv_point_kernel (conv_point.hpp): the input channels must be a
     // multiple of point_ic; 0 for the other kernels.
     int point_ic = 0;
     // conv_point_split_kernel: split convs only, all splits in one workgroup.
     bool point_split = false;
-    // Measured cost (see plan_cost in conv_igemm.hip), or all zero.
+    // Measured cost (measured_cost in conv_igemm.hip), or all zero.
     float cost[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     // Row staging of widths that are no multiple of 8: even, odd (or null:
     // such widths are staged pixel by pixel, by launch_scalar).

@@ -76,7 +76,10 @@ struct WsCfg {
     static constexpr int STAGE_BATCH = MT * NT * 16 + RING * MT * 4 > 160 ? 1 : 2;
     static_assert(MTT % WAVES == 0 && MT >= 1 && BN % 32 == 0 && TW % 8 == 0 && SC % 16 == 0, "tile shape");
     static_assert(S == 1 || S == 2, "stride");
-    static_assert(TAPS % RING == 0, "ring slots are static per tap");
+    // Ring slots are static per unrolled step: a ring of up to one 16-channel
+    // step divides its nine taps, a deeper one is that many whole steps.
+    static constexpr int RSTEPS = RING > TAPS ? RING / TAPS : 1;
+    static_assert(TAPS % RING == 0 || (RING % TAPS == 0 && (SC / 16) % RSTEPS == 0), "ring slots are static per step");
     static_assert(LDS * 2 * OCC <= 160 * 1024, "LDS budget");
     static_assert(NP_PER_T <= UNITS_PER_T * 8, "channel-last staging registers");
     static constexpr bool NHWC_EPI = BN * EPI_ROW_N <= LDS, NHWC_D2S_EPI = 4 * BN * EPI_ROW_D <= LDS;
@@ -232,7 +235,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
 #pragma unroll
     for (int s = 0; s < C::RING; ++s)
 #pragma unroll
-        for (int mt = 0; mt < C::MT; ++mt) ring[s][mt] = frag(s, mt);
+        for (int mt = 0; mt < C::MT; ++mt) ring[s][mt] = frag(min(s, total - 1), mt);
     floatx16 acc[C::MT][C::NT];
 #pragma unroll
     for (int mt = 0; mt < C::MT; ++mt)
@@ -269,8 +272,9 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
     u32x4 pv[C::UNITS_PER_T][8];
     std::uint32_t poff[C::UNITS_PER_T];
     int cb_next = 0;  // channel-last: first channel of the pass being loaded
-    auto kstep = [&](int c16, int tap, int coff, int boff, bool pipe_issue) {
+    auto kstep = [&](int c16, int tap, int coff, int boff, bool pipe_issue, int sub = 0) {
         const int s = c16 * C::TAPS + tap;
+        const int slot = (sub * C::TAPS + tap) % C::RING;
         const int ky = tap / C::KW, kx = tap % C::KW;
         half8 bv[C::NT];
 #pragma unroll
@@ -279,8 +283,8 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
         half8 av[C::MT];
 #pragma unroll
         for (int mt = 0; mt < C::MT; ++mt) {
-            av[mt] = __builtin_bit_cast(half8, ring[tap % C::RING][mt]);
-            ring[tap % C::RING][mt] = frag(min(s + C::RING, total - 1), mt);
+            av[mt] = __builtin_bit_cast(half8, ring[slot][mt]);
+            ring[slot][mt] = frag(min(s + C::RING, total - 1), mt);
         }
         if (C::PIPE && pipe_issue) {
             if (a.in_nhwc) {
@@ -352,9 +356,21 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
                 __syncthreads();
             }
             const int c16_end = min(nsteps16, (cb + C::SC) / 16);
-            for (int c16 = cb / 16; c16 < c16_end; ++c16) {
+            if constexpr (C::RSTEPS == 1) {
+                for (int c16 = cb / 16; c16 < c16_end; ++c16) {
 #pragma unroll
-                for (int tap = 0; tap < C::TAPS; ++tap) kstep(c16, tap, c16 * 16 - cb, 0, false);
+                    for (int tap = 0; tap < C::TAPS; ++tap) kstep(c16, tap, c16 * 16 - cb, 0, false);
+                }
+            } else {
+                // Whole rings of RSTEPS 16-channel steps (the host runs these
+                // variants on multiples of 16 RSTEPS channels only: a test
+                // inside the ring would make every load wait at its join).
+                for (int c0 = cb / 16; c0 < c16_end; c0 += C::RSTEPS) {
+#pragma unroll
+                    for (int sub = 0; sub < C::RSTEPS; ++sub)
+#pragma unroll
+                        for (int tap = 0; tap < C::TAPS; ++tap) kstep(c0 + sub, tap, (c0 + sub) * 16 - cb, 0, false, sub);
+                }
             }
         }
     }
@@ -538,6 +554,7 @@ constexpr Variant with_ragged_ws(Variant v)
     v.launch_scalar = &launch_mfma<Cfg<C::BM, C::TH, C::TW, 3, 3, C::S, 16, 0, false, C::WAVES, 1, 1>>;
     v.launch_rag[0] = &launch_ws<C, 1>;
     v.launch_rag[1] = &launch_ws<C, 2>;
+    v.ws_mult = 16 * C::RSTEPS;
     return v;
 }
 
