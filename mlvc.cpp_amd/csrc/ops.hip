@@ -19,14 +19,14 @@
 //     steps, exponent-bit scaling), kernels_x86_avx2.cpp:30-62.
 //
 // These kernels are HBM-bound: each thread moves 8 consecutive FP16 values
-// of a plane (16-byte accesses when planes are multiples of 8 and buffers
-// 16-byte aligned), and a grid-stride loop covers the planes.
+// of a plane in one 16-byte access, and a grid-stride loop covers the planes.
 
 #include "common.hpp"
 #include "mlvc_hip_device.h"
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -70,24 +70,35 @@ __device__ __forceinline__ float exp_lane(float x)
 __device__ __forceinline__ float sigmoid(float x) { return 1.0f / keep(1.0f + exp_lane(keep(0.0f - x))); }
 
 // Eight consecutive FP16 values of a plane; n < 8 only at a plane's end.
-template <bool VEC>
+// VEC: on 16 bytes. Otherwise (planes of a length that is no multiple of 8,
+// operands off 16 bytes) still one 16-byte access, which gfx950 allows on any
+// element: element by element, planes of 135x241 ran at half the rate (tails
+// of 64 channels 93 -> 50 us, feature update of 48 channels 15.7 -> 8.4 us).
+// NT: non-temporal, for launches that move more than the MALL holds.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+template <bool VEC, bool NT = false>
 __device__ __forceinline__ void ld8(const u16* p, int n, u16 (&v)[8])
 {
-    if (VEC && n == 8) {
-        const uint4 q = *reinterpret_cast<const uint4*>(p);
+    if (n == 8) {
+        using A = std::conditional_t<VEC, u32x4, u32x4_any>;
+        u32x4 q;
+        if constexpr (NT) q = __builtin_nontemporal_load(reinterpret_cast<const A*>(p));
+        else q = *reinterpret_cast<const A*>(p);
         __builtin_memcpy(v, &q, 16);
     } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = j < n ? p[j] : u16{0};
     }
 }
-template <bool VEC>
+template <bool VEC, bool NT = false>
 __device__ __forceinline__ void st8(u16* p, int n, const u16 (&v)[8])
 {
-    if (VEC && n == 8) {
-        uint4 q;
+    if (n == 8) {
+        using A = std::conditional_t<VEC, u32x4, u32x4_any>;
+        u32x4 q;
         __builtin_memcpy(&q, v, 16);
-        *reinterpret_cast<uint4*>(p) = q;
+        if constexpr (NT) __builtin_nontemporal_store(q, reinterpret_cast<A*>(p));
+        else *reinterpret_cast<A*>(p) = q;
     } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
@@ -335,7 +346,7 @@ __device__ __forceinline__ float gate(const u16* lut, u16 h)
 
 constexpr int kFeatureBlock = 1024;
 
-template <bool VEC>
+template <bool VEC, bool NT>
 __global__ __launch_bounds__(kFeatureBlock) void feature_kernel(const u16* __restrict__ x, const u16* __restrict__ hist,
                                                                 const u16* __restrict__ scale, u16* __restrict__ feature,
                                                                 u16* __restrict__ scaled_out, u16* __restrict__ blended_out, int n,
@@ -351,10 +362,10 @@ __global__ __launch_bounds__(kFeatureBlock) void feature_kernel(const u16* __res
         const size_t p0 = (t % p8) * 8, plane = t / p8, c = plane % ch, b = plane / ch;
         const int cnt = static_cast<int>(std::min<size_t>(8, hw - p0));
         u16 va[8], vb[8], vc[8], vh[8], so[8], bo[8];
-        ld8<VEC>(x + (b * 3 * ch + c) * hw + p0, cnt, va);
-        ld8<VEC>(x + (b * 3 * ch + ch + c) * hw + p0, cnt, vb);
-        ld8<VEC>(x + (b * 3 * ch + 2 * ch + c) * hw + p0, cnt, vc);
-        ld8<VEC>(hist + plane * hw + p0, cnt, vh);
+        ld8<VEC, NT>(x + (b * 3 * ch + c) * hw + p0, cnt, va);
+        ld8<VEC, NT>(x + (b * 3 * ch + ch + c) * hw + p0, cnt, vb);
+        ld8<VEC, NT>(x + (b * 3 * ch + 2 * ch + c) * hw + p0, cnt, vc);
+        ld8<VEC, NT>(hist + plane * hw + p0, cnt, vh);
         const float s = h2f(scale[c]);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -367,10 +378,10 @@ __global__ __launch_bounds__(kFeatureBlock) void feature_kernel(const u16* __res
             const float gated = r16(sc * h2f(bo[j]));
             so[j] = rnd(gated * s);
         }
-        st8<VEC>(feature + (b * 2 * ch + c) * hw + p0, cnt, so);
-        st8<VEC>(feature + (b * 2 * ch + ch + c) * hw + p0, cnt, bo);
-        if (scaled_out) st8<VEC>(scaled_out + plane * hw + p0, cnt, so);
-        if (blended_out) st8<VEC>(blended_out + plane * hw + p0, cnt, bo);
+        st8<VEC, NT>(feature + (b * 2 * ch + c) * hw + p0, cnt, so);
+        st8<VEC, NT>(feature + (b * 2 * ch + ch + c) * hw + p0, cnt, bo);
+        if (scaled_out) st8<VEC, NT>(scaled_out + plane * hw + p0, cnt, so);
+        if (blended_out) st8<VEC, NT>(blended_out + plane * hw + p0, cnt, bo);
     }
 }
 
@@ -382,7 +393,7 @@ __global__ __launch_bounds__(kFeatureBlock) void feature_kernel(const u16* __res
 //   y_raw[q] = fp16(rne(fp16(s[q] + s[q+Q]))),
 //   upd = fp16(fp16(y_raw + tail) * update_scale{0,1}),
 //   concat2 = upd, concat3 [N, 6Q, HW] = upd | prior.
-template <bool VEC>
+template <bool VEC, bool NT>
 __global__ __launch_bounds__(kBlock) void y0_tail_kernel(mlvc_hip_y0_tail_desc d)
 {
     const size_t hw = d.hw, q = static_cast<size_t>(d.q), p8 = (hw + 7) / 8, total = static_cast<size_t>(d.n) * q * p8;
@@ -406,10 +417,10 @@ __global__ __launch_bounds__(kBlock) void y0_tail_kernel(mlvc_hip_y0_tail_desc d
             u16 (&vh)[8] = pv[h];
             u16 (&vt)[8] = pv[2 + h];
             u16 vl[8], vq[8], cl[8], nr[8];
-            ld8<VEC>(prior + (b * 4 * q + cc) * hw + p0, cnt, vh);
-            ld8<VEC>(prior + (b * 4 * q + 2 * q + cc) * hw + p0, cnt, vt);
-            ld8<VEC>(latent + (b * 2 * q + cc) * hw + p0, cnt, vl);
-            ld8<VEC>(qs + (b * 2 * q + cc) * hw + p0, cnt, vq);
+            ld8<VEC, NT>(prior + (b * 4 * q + cc) * hw + p0, cnt, vh);
+            ld8<VEC, NT>(prior + (b * 4 * q + 2 * q + cc) * hw + p0, cnt, vt);
+            ld8<VEC, NT>(latent + (b * 2 * q + cc) * hw + p0, cnt, vl);
+            ld8<VEC, NT>(qs + (b * 2 * q + cc) * hw + p0, cnt, vq);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 cl[j] = rnd(maxps(h2f(vh[j]), d.clip_min));
@@ -419,32 +430,32 @@ __global__ __launch_bounds__(kBlock) void y0_tail_kernel(mlvc_hip_y0_tail_desc d
                 const float diff = r16(h2f(nr[j]) - tl[h][j]);
                 sv[h][j] = r16(diff * h2f(vq[j]));
             }
-            st8<VEC>(normalized + (b * 2 * q + cc) * hw + p0, cnt, nr);
-            st8<VEC>(clipped + (b * 2 * q + cc) * hw + p0, cnt, cl);
+            st8<VEC, NT>(normalized + (b * 2 * q + cc) * hw + p0, cnt, nr);
+            st8<VEC, NT>(clipped + (b * 2 * q + cc) * hw + p0, cnt, cl);
         }
         u16 raw[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) raw[j] = rnd(__builtin_rintf(r16(sv[0][j] + sv[1][j])));
-        st8<VEC>(y_raw + (b * q + qc) * hw + p0, cnt, raw);
+        st8<VEC, NT>(y_raw + (b * q + qc) * hw + p0, cnt, raw);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const size_t cc = qc + h * q;
             u16 vu[8], up[8];
-            ld8<VEC>(us[h] + (b * q + qc) * hw + p0, cnt, vu);
+            ld8<VEC, NT>(us[h] + (b * q + qc) * hw + p0, cnt, vu);
 #pragma unroll
             for (int j = 0; j < 8; ++j) up[j] = rnd(r16(h2f(raw[j]) + tl[h][j]) * h2f(vu[j]));
-            st8<VEC>(concat2 + (b * 2 * q + cc) * hw + p0, cnt, up);
-            st8<VEC>(concat3 + (b * 6 * q + cc) * hw + p0, cnt, up);
+            st8<VEC, NT>(concat2 + (b * 2 * q + cc) * hw + p0, cnt, up);
+            st8<VEC, NT>(concat3 + (b * 6 * q + cc) * hw + p0, cnt, up);
         }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) st8<VEC>(concat3 + (b * 6 * q + 2 * q + qc + k * q) * hw + p0, cnt, pv[k]);
+        for (int k = 0; k < 4; ++k) st8<VEC, NT>(concat3 + (b * 6 * q + 2 * q + qc + k * q) * hw + p0, cnt, pv[k]);
     }
 }
 
 //   s = fp16(fp16(normalized - prior) * quant_scale), y_raw as above,
 //   upd = fp16(fp16(y_raw + prior) * update_scale{0,1}),
 //   out = fp16(fp16(concat2 + upd) * clipped).
-template <bool VEC>
+template <bool VEC, bool NT>
 __global__ __launch_bounds__(kBlock) void y1_tail_kernel(mlvc_hip_y1_tail_desc d)
 {
     const size_t hw = d.hw, q = static_cast<size_t>(d.q), p8 = (hw + 7) / 8, total = static_cast<size_t>(d.n) * q * p8;
@@ -464,9 +475,9 @@ __global__ __launch_bounds__(kBlock) void y1_tail_kernel(mlvc_hip_y1_tail_desc d
         for (int h = 0; h < 2; ++h) {
             const size_t off = (b * 2 * q + qc + h * q) * hw + p0;
             u16 vn[8], vp[8], vq[8];
-            ld8<VEC>(normalized + off, cnt, vn);
-            ld8<VEC>(prior + off, cnt, vp);
-            ld8<VEC>(qs + off, cnt, vq);
+            ld8<VEC, NT>(normalized + off, cnt, vn);
+            ld8<VEC, NT>(prior + off, cnt, vp);
+            ld8<VEC, NT>(qs + off, cnt, vq);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 pr[h][j] = h2f(vp[j]);
@@ -476,23 +487,39 @@ __global__ __launch_bounds__(kBlock) void y1_tail_kernel(mlvc_hip_y1_tail_desc d
         u16 raw[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) raw[j] = rnd(__builtin_rintf(r16(sv[0][j] + sv[1][j])));
-        st8<VEC>(y_raw + (b * q + qc) * hw + p0, cnt, raw);
+        st8<VEC, NT>(y_raw + (b * q + qc) * hw + p0, cnt, raw);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const size_t off = (b * 2 * q + qc + h * q) * hw + p0;
             u16 vu[8], v2[8], vc[8], o[8];
-            ld8<VEC>(us[h] + (b * q + qc) * hw + p0, cnt, vu);
-            ld8<VEC>(concat2 + off, cnt, v2);
-            ld8<VEC>(clipped + off, cnt, vc);
+            ld8<VEC, NT>(us[h] + (b * q + qc) * hw + p0, cnt, vu);
+            ld8<VEC, NT>(concat2 + off, cnt, v2);
+            ld8<VEC, NT>(clipped + off, cnt, vc);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float upd = r16(r16(h2f(raw[j]) + pr[h][j]) * h2f(vu[j]));
                 const float add = r16(h2f(v2[j]) + upd);
                 o[j] = rnd(add * h2f(vc[j]));
             }
-            st8<VEC>(out + off, cnt, o);
+            st8<VEC, NT>(out + off, cnt, o);
         }
     }
+}
+
+// Whether a launch of `bytes` streams past the caches: more than the 256 MB
+// MALL holds, so what it reads and writes is not found there by the next
+// launch either way. Non-temporal accesses then leave room for the lines still
+// to be merged: feature update of 64 channels at 544x960 (401 MB) 85 -> 80 us,
+// both tails of 96 channels at 272x480 (852 MB) 183 -> 167 us. Launches that
+// fit keep ordinary accesses, whose results the next launch finds in the MALL.
+bool streams(std::size_t bytes) { return bytes > (std::size_t{256} << 20); }
+
+// go(vec, nt) with both as compile-time constants.
+template <typename F>
+void by_access(bool vec, bool nt, F&& go)
+{
+    if (vec) nt ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+    else nt ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 void need(bool ok, const char* what)
@@ -700,12 +727,12 @@ int mlvc_hip_feature_update(const void* x, const void* history, const void* scal
         // blocks the device holds at once (two per CU) walks the work.
         const unsigned grid = static_cast<unsigned>(
             std::max<size_t>(1, std::min<size_t>((work + kFeatureBlock - 1) / kFeatureBlock, 2 * static_cast<size_t>(conv::cu_count()))));
-        if (vec)
-            hipLaunchKernelGGL(feature_kernel<true>, dim3(grid), dim3(kFeatureBlock), 0, to_stream(s), px, ph, pc, pf, ps, pb, n,
-                               channels, hw);
-        else
-            hipLaunchKernelGGL(feature_kernel<false>, dim3(grid), dim3(kFeatureBlock), 0, to_stream(s), px, ph, pc, pf, ps, pb, n,
-                               channels, hw);
+        // Three planes of x, the history, two planes out (and again where the outputs are split).
+        const std::size_t bytes = static_cast<std::size_t>(n) * channels * hw * 2 * (scaled ? 8 : 6);
+        by_access(vec, streams(bytes), [&](auto v, auto nt) {
+            hipLaunchKernelGGL((feature_kernel<v.value, nt.value>), dim3(grid), dim3(kFeatureBlock), 0, to_stream(s), px, ph, pc, pf,
+                               ps, pb, n, channels, hw);
+        });
         check(hipGetLastError(), "feature_update launch");
     });
 }
@@ -721,8 +748,10 @@ int mlvc_hip_y0_tail(const mlvc_hip_y0_tail_desc* d, mlvc_hip_stream s)
         bool vec = d->hw % 8 == 0;
         for (const void* p : ptrs) vec = vec && aligned16(p);
         const size_t work = static_cast<size_t>(d->n) * d->q * ((d->hw + 7) / 8);
-        if (vec) launch(y0_tail_kernel<true>, work, to_stream(s), *d);
-        else launch(y0_tail_kernel<false>, work, to_stream(s), *d);
+        // 10 q planes read, 13 q written.
+        const std::size_t bytes = static_cast<std::size_t>(d->n) * d->q * d->hw * 2 * 23;
+        by_access(vec, streams(bytes),
+                  [&](auto v, auto nt) { launch(y0_tail_kernel<v.value, nt.value>, work, to_stream(s), *d); });
     });
 }
 
@@ -737,8 +766,10 @@ int mlvc_hip_y1_tail(const mlvc_hip_y1_tail_desc* d, mlvc_hip_stream s)
         bool vec = d->hw % 8 == 0;
         for (const void* p : ptrs) vec = vec && aligned16(p);
         const size_t work = static_cast<size_t>(d->n) * d->q * ((d->hw + 7) / 8);
-        if (vec) launch(y1_tail_kernel<true>, work, to_stream(s), *d);
-        else launch(y1_tail_kernel<false>, work, to_stream(s), *d);
+        // 12 q planes read, 3 q written.
+        const std::size_t bytes = static_cast<std::size_t>(d->n) * d->q * d->hw * 2 * 15;
+        by_access(vec, streams(bytes),
+                  [&](auto v, auto nt) { launch(y1_tail_kernel<v.value, nt.value>, work, to_stream(s), *d); });
     });
 }
 
