@@ -121,7 +121,7 @@ typedef struct mlvc_hip_conv_desc {
     int in_nhwc, out_nhwc;
 } mlvc_hip_conv_desc;
 
-/* Chooses the kernel variant for the geometry by a cost model (sets
+/* Chooses the kernel variant for the geometry by its measured cost (sets
  * desc->variant and desc->vector_io). Every 3x3 variant accumulates in the
  * same K order, and so does every 1x1 variant, so the choice never changes
  * results. Role of the reference's per-shape tile choice by fixed thresholds
@@ -137,11 +137,12 @@ typedef struct mlvc_hip_conv_desc {
  * ceil(ic / split_c) ranges of input channels, split_c = 64 * ceil(ic /
  * (64 * s)), s = min(8, 512 / items, ic / 64) (integer division; no split
  * when s <= 1). Split s sums its channels in the usual K order into an FP32
- * partial (split 0 seeded with the bias, the others with zero); a second
- * kernel adds the partials in split order, rounds to FP16 and applies the
- * epilogue (ReGLU included) and the DEPTH_TO_SPACE store. Split convs run on
- * the conv_mfma variants only and need desc->workspace (FP32 partials,
- * mlvc_hip_conv_workspace_bytes; 16-byte aligned). The reference's role for
+ * partial (split 0 seeded with the bias, the others with zero); the partials
+ * are added in split order, rounded to FP16 and given the epilogue (ReGLU
+ * included) and the DEPTH_TO_SPACE store, by a second kernel or, in the
+ * mfma_ptk variants, in the workgroup that made them. Split convs run on the
+ * mfma variants only and need desc->workspace (FP32 partials,
+ * mlvc_hip_conv_workspace_bytes; 16-byte aligned), whichever it is. The reference's role for
  * this: its small-tile choice where a large-tile grid would be under two
  * waves of SMs (driver_cubin/src/execution_plan.cpp:379-391). */
 int mlvc_hip_conv_plan(mlvc_hip_conv_desc* desc);

@@ -12,8 +12,11 @@
 //   * the waves split the output channels (wave w owns m-tiles
 //     w*MT .. w*MT + MT - 1) and each streams its own A fragments (weights
 //     pre-packed in fragment order, [ocb][c16][tap][m-tile][lane][8]) from
-//     L2 straight into a register ring three steps deep, so weights never
-//     pass through LDS and no two waves of a workgroup fetch the same ones;
+//     L2 straight into a register ring (3, 9 or 18 steps deep), so weights
+//     never pass through LDS and no two waves of a workgroup fetch the same
+//     ones. With few workgroups the stream is a chain of L2 latencies one ring
+//     apart: 18 steps instead of 9 took 256->768 at 30x54 from 20.5 to 17.4 us;
+//     36 spill;
 //   * every wave covers all BN pixels, reading its B fragments from the
 //     staged halo;
 //   * two workgroups per CU (halo <= 80 KB, 128 accumulator registers), so
