@@ -525,7 +525,10 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             if (k.ws_ic && k.ws_mult > 16 && d.ic % k.ws_mult != 0)
                 throw std::runtime_error("conv: variant does not match the geometry");
             if (k.ws_ic && (d.x2 || a.s2d > 1)) throw std::runtime_error("conv: variant needs a plain input");
-            if (k.ws_ic && !vec && (even || !k.launch_scalar)) throw std::runtime_error("conv: variant needs 16-byte row staging");
+            // Operands without the alignment: the variants the plan chooses
+            // stage them pixel by pixel (NCHW).
+            if (k.ws_ic && !vec && !ragged && (!k.launch_scalar || d.in_nhwc || d.out_nhwc))
+                throw std::runtime_error("conv: variant needs 16-byte row staging");
             (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : ragged ? ragged : k.launch_scalar)(a, grid, to_stream(s));
             if (a.ksplit > 1 && !(k.point_split && vec)) {
                 ConvArgs r = a;  // the reduce works in the real output geometry

@@ -52,12 +52,12 @@ const Variant kTable[] = {
     MLVC_VARIANT_WSR(128, 8, 24, 64, 2, 9),
     MLVC_VARIANT_WSR(128, 4, 40, 64, 2, 9),
     MLVC_VARIANT_WSR(128, 4, 48, 64, 2, 9),
-    costed(MLVC_VARIANT_WS(128, 8, 32, 64, 2), 2.118f, 0.216f, 4.243f, 1.777f),
+    costed(with_scalar_ws<WsCfg<128, 8, 32, 64, 2>>(MLVC_VARIANT_WS(128, 8, 32, 64, 2)), 2.118f, 0.216f, 4.243f, 1.777f),
     // Two m-tiles per wave with a 9-step ring.
     MLVC_VARIANT_WSR(256, 4, 24, 64, 2, 9),
     MLVC_VARIANT_WSR(256, 2, 48, 64, 2, 9),
     // Pipelined passes of 32 channels.
-    costed(MLVC_VARIANT_WSP(256, 4, 32, 32, 2, 3), 2.936f, 0.292f, 0.731f, 2.101f),
+    costed(with_scalar_ws<WsCfg<256, 4, 32, 32, 2>>(MLVC_VARIANT_WSP(256, 4, 32, 32, 2, 3)), 2.936f, 0.292f, 0.731f, 2.101f),
     MLVC_VARIANT_WSP(128, 8, 32, 32, 2, 3),
     MLVC_VARIANT_WSP(128, 4, 32, 32, 2, 9),
     MLVC_VARIANT_WSP(128, 4, 48, 32, 2, 9),
@@ -81,7 +81,7 @@ const Variant kTable[] = {
     // 255 8x16 tiles x 2 channel blocks = 510 workgroups, where the 4x48
     // tiles' 680 take two rounds of 512 slots with the second a third full.
     // LDS for the channel-last DEPTH_TO_SPACE(2) output tile (72 KB).
-    costed(MLVC_VARIANT_WSPD(256, 8, 16, 32, 2, 3), 2.934f, 0.218f, 0.886f, 2.191f),
+    costed(with_scalar_ws<WsCfg<256, 8, 16, 32, 2>>(MLVC_VARIANT_WSPD(256, 8, 16, 32, 2, 3)), 2.934f, 0.218f, 0.886f, 2.191f),
 };
 }  // namespace
 

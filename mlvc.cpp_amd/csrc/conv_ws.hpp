@@ -547,14 +547,21 @@ void launch_ws(const ConvArgs& a, dim3 grid, hipStream_t s)
     hipLaunchKernelGGL((conv_ws_kernel<C, RAG>), grid, dim3(C::kThreads), 0, s, a);
 }
 
-// A variant that also runs NCHW rows of any width: the ragged builds, and for
-// operands without the alignment those need (x off 16 bytes, images off 4) the
-// per-pixel staging of conv_mfma_kernel on the same tile, whose packed weights
-// are the same.
+// A variant that also runs NCHW operands without the alignment 16-byte rows
+// need (x off 16 bytes): by the per-pixel staging of conv_mfma_kernel on the
+// same tile, whose packed weights are the same.
+template <class C>
+constexpr Variant with_scalar_ws(Variant v)
+{
+    v.launch_scalar = &launch_mfma<Cfg<C::BM, C::TH, C::TW, 3, 3, C::S, 16, 0, false, C::WAVES, 1, 1>>;
+    return v;
+}
+
+// ...and NCHW rows of any width, by the ragged builds.
 template <class C>
 constexpr Variant with_ragged_ws(Variant v)
 {
-    v.launch_scalar = &launch_mfma<Cfg<C::BM, C::TH, C::TW, 3, 3, C::S, 16, 0, false, C::WAVES, 1, 1>>;
+    v = with_scalar_ws<C>(v);
     v.launch_rag[0] = &launch_ws<C, 1>;
     v.launch_rag[1] = &launch_ws<C, 2>;
     v.ws_mult = 16 * C::RSTEPS;

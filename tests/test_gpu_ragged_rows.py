@@ -153,11 +153,23 @@ def test_row_staging_equals_pixel_staging(case):
             assert torch.equal(got.view(torch.int16), first.view(torch.int16)), f"{name}, rows={rows}"
 
 
-# Operands off 16 bytes keep running on ragged widths (per-pixel staging).
-@pytest.mark.parametrize("case", [CASES[3], CASES[12], CASES[16]], ids=("3x3", "3x3s2", "1x1"))
+# Operands off 16 bytes keep running, whatever the plan chooses: by per-pixel
+# staging. Every variant of the cost table either runs them, with the same
+# bits, or is one that no plan chooses and refuses them.
+UNALIGNED = [CASES[3], CASES[12], CASES[16], (1, 96, 12, 32, 192, 3, 1, 1, LRELU, 0, 0), (1, 128, 16, 32, 256, 3, 1, 1, LRELU, 2, 0),
+             (1, 64, 16, 48, 128, 3, 2, 1, RESIDUAL, 0, 0), (1, 128, 8, 16, 96, 1, 1, 0, LRELU, 0, 0)]
+COSTED = ("ws_bm128_8x32_k3x3_s1_sc64_occ2", "ws_bm256_4x32_k3x3_s1_sc32_occ2_r3_pipe", "ws_bm256_8x16_k3x3_s1_sc32_occ2_r3_pipe",
+          "ws_bm128_4x16_k3x3_s1_sc64_occ2_r18", "ws_bm64_2x32_k3x3_s1_sc64_occ4_w2_r9")
+
+
+@pytest.mark.parametrize("case", UNALIGNED, ids=lambda c: "n{}_ic{}_{}x{}_oc{}_k{}s{}p{}_e{}_d{}_c{}".format(*c))
 def test_unaligned_input_pointer(case):
     print(case, flush=True)
     lib, d, wt, b, keep, shape, (want, tol) = setup(case)
     aligned = run(lib, d, wt, b, shape, d.variant, 1)
+    buf, count = (C.c_int * 512)(), C.c_int()
+    assert lib.mlvc_hip_conv_candidates(C.byref(d), buf, 512, C.byref(count)) == 0
+    names = {lib.mlvc_hip_conv_variant_name(v).decode(): v for v in buf[:count.value]}
     lib, d, wt, b, keep, shape, _ = setup(case, offset=9)
-    assert torch.equal(run(lib, d, wt, b, shape, d.variant, 1).view(torch.int16), aligned.view(torch.int16))
+    for v in {d.variant, *(names[n] for n in COSTED if n in names)}:
+        assert torch.equal(run(lib, d, wt, b, shape, v, 1).view(torch.int16), aligned.view(torch.int16))
