@@ -261,9 +261,11 @@ bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
     // conv_point_kernel: whole passes of channels, pixel rows on 4 bytes, a
     // concat split on a 16-channel step, offsets below 2^31; no ReGLU. Its
     // split form: split convs of a plain input and up to eight splits (a wave
-    // each).
+    // each) of whole 64-channel halves.
     if (k.point_ic && (!flat || !flat_1x1(d) || d.ic % k.point_ic != 0 || iw % 2 != 0 || d.ic_split % 16 != 0 ||
-                       (d.ksplit > 1) != k.point_split || (k.point_split && (concat(d) || d.ksplit > 8)) || d.epilogue == MLVC_EPI_REGLU || static_cast<std::uint64_t>(d.ic) * iw * 2 >= (1ull << 31) ||
+                       (d.ksplit > 1) != k.point_split ||
+                       (k.point_split && (concat(d) || d.ksplit > 8 || d.split_c % k.point_ic != 0)) ||
+                       d.epilogue == MLVC_EPI_REGLU || static_cast<std::uint64_t>(d.ic) * iw * 2 >= (1ull << 31) ||
                        static_cast<std::uint64_t>((d.oc + k.bm - 1) / k.bm) * k.bm * d.ic * 2 >= (1ull << 31)))
         return false;
     return !(d.kh == 1 && flat != (k.th == 1));
@@ -468,7 +470,10 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
                                           d.ksplit > 1))
             throw std::runtime_error("conv: channel-last operands need a weight-streaming variant");
         if (d.ksplit > 1) {
-            if (k.bm == 0 || k.ws_ic || d.split_c <= 0 || d.split_c % k.kc != 0 ||
+            // Split K: tiles whose chunk divides the split; the 1x1 kernels
+            // take the splits the general kernel's 1x1 tiles take.
+            const int chunk = k.point_ic ? std::max(k.kc, 32) : k.kc;
+            if (k.bm == 0 || k.ws_ic || d.split_c <= 0 || d.split_c % chunk != 0 ||
                 static_cast<long long>(d.split_c) * (d.ksplit - 1) >= d.ic || static_cast<long long>(d.split_c) * d.ksplit < d.ic)
                 throw std::runtime_error("conv: split K needs a conv_mfma variant whose chunk divides the split");
             if (!d.workspace || d.workspace_bytes < mlvc_hip_conv_workspace_bytes(&d) ||
@@ -507,7 +512,10 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
                                (a.ksplit > 1) != k.point_split || (k.point_split && (d.x2 || a.ksplit > 8)) ||
                                (d.x2 && d.ic_split % 16 != 0) || d.epilogue == MLVC_EPI_REGLU))
                 throw std::runtime_error("conv: variant does not match the geometry");
-            const bool vec = rows && (even || k.point_ic);
+            // All splits in one workgroup: each wave multiplies whole
+            // 64-channel halves. Other splits sum through memory.
+            const bool halves = !k.point_split || a.split_c % k.point_ic == 0;
+            const bool vec = rows && (even || k.point_ic) && halves;
             const auto ragged = rows && !even && images4 ? k.launch_rag[a.iw & 1] : nullptr;
             a.tiles_x = (a.ow + k.tw - 1) / k.tw;
             a.nchunks = (d.ic + k.kc - 1) / k.kc;

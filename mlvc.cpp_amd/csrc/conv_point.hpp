@@ -287,7 +287,9 @@ void launch_point(const ConvArgs& a, dim3 grid, hipStream_t s)
 // partials meet in LDS, and the waves add them in split order, round and apply
 // the epilogue: the sums of conv_mfma_kernel's split and
 // conv_splitk_reduce_kernel, bit for bit, without the partials' trip through
-// memory and the second launch. Few pixels and many channels are bound by
+// memory and the second launch. Splits are whole 64-channel halves: both are
+// multiplied whole, so the host sends other splits (set by hand; the plan's
+// are multiples of 64) to the two kernels. Few pixels and many channels are bound by
 // latency, so each wave has 128 channels of X (DMA into LDS of its own, no
 // barrier) and W in flight at once; with the usual split_c of 128 that is its
 // whole share. 1024->256 at 23x40, 8 splits: 16.7 us in two kernels, 5.8 here.
@@ -430,8 +432,9 @@ void launch_point_split(const ConvArgs& a, dim3, hipStream_t s)
                        static_cast<unsigned>(a.ksplit * C::WAVE * 2), s, a);
 }
 
-// Variant entry: weights packed with kc = 16. Operands off 16 bytes run the
-// split and the reduce kernel of conv_mfma_kernel on the same tile.
+// Variant entry: weights packed with kc = 16. Operands off 16 bytes and
+// splits off 64 channels run the split of conv_mfma_kernel on the same tile
+// and the reduce kernel.
 template <class C>
 constexpr Variant point_split_variant(const char* name)
 {

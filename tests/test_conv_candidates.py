@@ -104,6 +104,19 @@ def test_split_rule():
     assert plan(1024, 46, 80, 256, 1, 1, pad=0, n=16)[0].ksplit <= 1
 
 
+def test_split_in_one_workgroup_takes_whole_halves_only():
+    """The variants that keep all splits in one workgroup multiply 64 channels
+    at a time: splits set by hand list them only in multiples of 64."""
+    for ksplit, split_c, want in ((8, 128, True), (4, 256, True), (16, 64, False), (7, 160, False), (6, 192, True), (11, 96, False),
+                                  (13, 80, False)):
+        d, _ = plan(1024, 23, 40, 256, 1, 1, pad=0)
+        d.ksplit, d.split_c = ksplit, split_c
+        names = candidates(1024, 23, 40, 256, 1, 1, pad=0, desc=d)
+        assert any(n.startswith("mfma_ptk") for n in names) == want, (ksplit, split_c, names)
+        # The general tiles take every split of whole 32-channel chunks.
+        assert any(n.startswith("mfma_bm") for n in names) == (split_c % 32 == 0), (ksplit, split_c, names)
+
+
 # The tuned convs of the 1920x1088 graph: (launch, ic, h, w, oc, stride,
 # DEPTH_TO_SPACE block, channel-last input, channel-last output).
 TUNED_1920 = [

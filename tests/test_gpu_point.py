@@ -79,3 +79,29 @@ def test_extreme_values():
         nan = torch.isnan(want)
         assert torch.equal(torch.isnan(got), nan)
         assert torch.equal(got[~nan].view(torch.int16), want[~nan].view(torch.int16))
+
+
+# (case, ksplit, split_c): splits set by hand, as a tuner of its own sets them.
+# The kernel that keeps all splits in one workgroup multiplies 64 channels at a
+# time; other splits (a last half of 32 channels) sum through memory.
+HAND_SPLITS = [((1, 1024, 23, 40, 256, 1, 1, 0, LRELU, 0, 0), 7, 160), ((1, 1024, 5, 34, 96, 1, 1, 0, RESIDUAL, 0, 0), 8, 128),
+               ((2, 768, 3, 22, 64, 1, 1, 0, NONE, 0, 0), 8, 96), ((1, 640, 5, 8, 33, 1, 1, 0, CLAMP, 0, 0), 2, 320)]
+
+
+@pytest.mark.parametrize("case,ksplit,split_c", HAND_SPLITS, ids=lambda v: str(v))
+def test_splits_set_by_hand(case, ksplit, split_c):
+    """A planned descriptor runs them with its variant; the sums are those of a general tile's two kernels."""
+    print(case, ksplit, split_c, flush=True)
+    lib, d, wt, b, keep, shape, (want, tol) = rows.setup(case)
+    d.ksplit, d.split_c = ksplit, split_c
+    ws = torch.empty(lib.mlvc_hip_conv_workspace_bytes(C.byref(d)), dtype=torch.uint8, device="cuda")
+    d.workspace, d.workspace_bytes = ws.data_ptr(), ws.numel()
+    assert lib.mlvc_hip_conv_variant_name(d.variant).decode().startswith("mfma_ptk")
+    buf, count = (C.c_int * 512)(), C.c_int()
+    assert lib.mlvc_hip_conv_candidates(C.byref(d), buf, 512, C.byref(count)) == 0
+    first = rows.run(lib, d, wt, b, shape, buf[0], 0)
+    assert lib.mlvc_hip_conv_variant_name(buf[0]).decode().startswith("mfma_bm")
+    assert ((first.double() - want).abs() / tol).max().item() <= 1.0
+    for v in {d.variant, *buf[:count.value]}:
+        for staging in (1, 0):
+            assert torch.equal(rows.run(lib, d, wt, b, shape, v, staging).view(torch.int16), first.view(torch.int16))
