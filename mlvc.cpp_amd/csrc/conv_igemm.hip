@@ -502,8 +502,9 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             const bool rows = d.vector_io && aligned && a.s2d <= 1 && (!a.x2 || a.ic_split % k.kc == 0) &&
                               (static_cast<std::uint64_t>(d.ic) + k.kc) * plane_bytes < (1ull << 31);
             // Rows of a multiple of 8 pixels (for the weight-streaming kernel,
-            // output rows too); else the ragged builds, whose buffer loads
-            // need every image's first element on 4 bytes.
+            // output rows too); else the ragged builds, which read NCHW rows
+            // and whose buffer loads need every image's first element on 4
+            // bytes.
             const bool even = a.iw % 8 == 0 && (!k.ws_ic || a.ow % 8 == 0);
             const std::uint64_t plane = static_cast<std::uint64_t>(a.ih) * a.iw;
             const bool images4 = d.n == 1 || ((a.x2 ? a.ic_split : d.ic) * plane % 2 == 0 &&
@@ -516,7 +517,8 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             // 64-channel halves. Other splits sum through memory.
             const bool halves = !k.point_split || a.split_c % k.point_ic == 0;
             const bool vec = rows && (even || k.point_ic) && halves;
-            const auto ragged = rows && !even && images4 ? k.launch_rag[a.iw & 1] : nullptr;
+            const bool nchw = !d.in_nhwc && !d.out_nhwc;
+            const auto ragged = rows && !even && images4 && nchw ? k.launch_rag[a.iw & 1] : nullptr;
             a.tiles_x = (a.ow + k.tw - 1) / k.tw;
             a.nchunks = (d.ic + k.kc - 1) / k.kc;
             a.tiles = a.tiles_x * ((a.oh + k.th - 1) / k.th);
@@ -535,7 +537,7 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             if (k.ws_ic && (d.x2 || a.s2d > 1)) throw std::runtime_error("conv: variant needs a plain input");
             // Operands without the alignment: the variants the plan chooses
             // stage them pixel by pixel (NCHW).
-            if (k.ws_ic && !vec && !ragged && (!k.launch_scalar || d.in_nhwc || d.out_nhwc))
+            if (k.ws_ic && !vec && !ragged && (!k.launch_scalar || !nchw))
                 throw std::runtime_error("conv: variant needs 16-byte row staging");
             (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : ragged ? ragged : k.launch_scalar)(a, grid, to_stream(s));
             if (a.ksplit > 1 && !(k.point_split && vec)) {

@@ -117,6 +117,23 @@ def test_split_in_one_workgroup_takes_whole_halves_only():
         assert any(n.startswith("mfma_bm") for n in names) == (split_c % 32 == 0), (ksplit, split_c, names)
 
 
+def test_ragged_rows_of_channel_last_operands_are_refused():
+    """The ragged builds read NCHW rows: a descriptor planned onto a variant
+    that has them and then given a channel-last operand is refused before
+    anything is launched, at every width that is no multiple of 8."""
+    lib = mlvc_hip.device_lib()
+    lib.mlvc_hip_last_error.restype = C.c_char_p
+    for ic, h, w, oc, stride in ((256, 30, 54, 768, 1), (64, 40, 23, 64, 1), (128, 40, 40, 192, 2), (64, 21, 62, 128, 2)):
+        for cl_in, cl_out in ((1, 0), (0, 1), (1, 1)):
+            d, _ = plan(ic, h, w, oc, stride=stride)
+            assert lib.mlvc_hip_conv_variant_name(d.variant).decode().startswith("ws_")
+            d.in_nhwc, d.out_nhwc = cl_in, cl_out
+            d.x = d.y = d.packed_w = d.bias = 4096  # never read: the launch fails on the host
+            assert lib.mlvc_hip_conv_launch(C.byref(d), None) == -1
+            msg = lib.mlvc_hip_last_error().decode()
+            assert "row staging" in msg or "channel-last operands" in msg, (ic, w, stride, cl_in, cl_out, msg)
+
+
 # The tuned convs of the 1920x1088 graph: (launch, ic, h, w, oc, stride,
 # DEPTH_TO_SPACE block, channel-last input, channel-last output).
 TUNED_1920 = [
