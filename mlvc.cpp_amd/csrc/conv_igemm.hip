@@ -516,9 +516,15 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             // All splits in one workgroup: each wave multiplies whole
             // 64-channel halves. Other splits sum through memory.
             const bool halves = !k.point_split || a.split_c % k.point_ic == 0;
-            const bool vec = rows && (even || k.point_ic) && halves;
+            // The weight-streaming kernel's epilogue has no ReGLU and no
+            // DEPTH_TO_SPACE past 2 (a descriptor can get them after its
+            // plan): the general kernel has, on the same packed weights.
+            const bool epilogue = !k.ws_ic || (d.epilogue != MLVC_EPI_REGLU && a.d2s <= 2);
+            if (d.epilogue == MLVC_EPI_REGLU && k.bm % 64 != 0)
+                throw std::runtime_error("conv: ReGLU needs a variant of whole 64-channel blocks");
+            const bool vec = rows && (even || k.point_ic) && halves && epilogue;
             const bool nchw = !d.in_nhwc && !d.out_nhwc;
-            const auto ragged = rows && !even && images4 && nchw ? k.launch_rag[a.iw & 1] : nullptr;
+            const auto ragged = rows && !even && images4 && nchw && epilogue ? k.launch_rag[a.iw & 1] : nullptr;
             a.tiles_x = (a.ow + k.tw - 1) / k.tw;
             a.nchunks = (d.ic + k.kc - 1) / k.kc;
             a.tiles = a.tiles_x * ((a.oh + k.th - 1) / k.th);
@@ -538,7 +544,8 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             // Operands without the alignment: the variants the plan chooses
             // stage them pixel by pixel (NCHW).
             if (k.ws_ic && !vec && !ragged && (!k.launch_scalar || !nchw))
-                throw std::runtime_error("conv: variant needs 16-byte row staging");
+                throw std::runtime_error(epilogue ? "conv: variant needs 16-byte row staging"
+                                                  : "conv: variant does not run the epilogue or the depth_to_space block");
             (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : ragged ? ragged : k.launch_scalar)(a, grid, to_stream(s));
             if (a.ksplit > 1 && !(k.point_split && vec)) {
                 ConvArgs r = a;  // the reduce works in the real output geometry
