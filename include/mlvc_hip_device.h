@@ -144,7 +144,14 @@ typedef struct mlvc_hip_conv_desc {
  * mfma variants only and need desc->workspace (FP32 partials,
  * mlvc_hip_conv_workspace_bytes; 16-byte aligned), whichever it is. The reference's role for
  * this: its small-tile choice where a large-tile grid would be under two
- * waves of SMs (driver_cubin/src/execution_plan.cpp:379-391). */
+ * waves of SMs (driver_cubin/src/execution_plan.cpp:379-391).
+ *
+ * A descriptor may change after its plan (another size, epilogue, fusion or
+ * split; 1x1 splits in multiples of 32 channels) if its weights are packed for
+ * the change: a planned variant runs it by the general kernel where its own
+ * cannot, with the same results. Planned for what it runs, it is faster. Not
+ * so: the kernel size and stride, the layouts, and ReGLU on a variant of
+ * 32-channel blocks, which are refused. */
 int mlvc_hip_conv_plan(mlvc_hip_conv_desc* desc);
 /* Bytes of FP32 partials a launch of desc needs (0 when not split). */
 size_t mlvc_hip_conv_workspace_bytes(const mlvc_hip_conv_desc* desc);

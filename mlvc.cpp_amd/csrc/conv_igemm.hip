@@ -473,7 +473,7 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             // Split K: tiles whose chunk divides the split; the 1x1 kernels
             // take the splits the general kernel's 1x1 tiles take.
             const int chunk = k.point_ic ? std::max(k.kc, 32) : k.kc;
-            if (k.bm == 0 || k.ws_ic || d.split_c <= 0 || d.split_c % chunk != 0 ||
+            if (k.bm == 0 || (k.ws_ic && !k.launch_scalar) || d.split_c <= 0 || d.split_c % chunk != 0 ||
                 static_cast<long long>(d.split_c) * (d.ksplit - 1) >= d.ic || static_cast<long long>(d.split_c) * d.ksplit < d.ic)
                 throw std::runtime_error("conv: split K needs a conv_mfma variant whose chunk divides the split");
             if (!d.workspace || d.workspace_bytes < mlvc_hip_conv_workspace_bytes(&d) ||
@@ -509,22 +509,27 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             const std::uint64_t plane = static_cast<std::uint64_t>(a.ih) * a.iw;
             const bool images4 = d.n == 1 || ((a.x2 ? a.ic_split : d.ic) * plane % 2 == 0 &&
                                               (!a.x2 || (d.ic - a.ic_split) * plane % 2 == 0));
-            if (k.point_ic && (a.ih != 1 || d.ic % k.point_ic != 0 || a.iw % 2 != 0 || a.s2d > 1 || a.d2s > 1 ||
-                               (a.ksplit > 1) != k.point_split || (k.point_split && (d.x2 || a.ksplit > 8)) ||
-                               (d.x2 && d.ic_split % 16 != 0) || d.epilogue == MLVC_EPI_REGLU))
-                throw std::runtime_error("conv: variant does not match the geometry");
-            // All splits in one workgroup: each wave multiplies whole
-            // 64-channel halves. Other splits sum through memory.
-            const bool halves = !k.point_split || a.split_c % k.point_ic == 0;
-            // The weight-streaming kernel's epilogue has no ReGLU and no
-            // DEPTH_TO_SPACE past 2 (a descriptor can get them after its
-            // plan): the general kernel has, on the same packed weights.
-            const bool epilogue = !k.ws_ic || (d.epilogue != MLVC_EPI_REGLU && a.d2s <= 2);
-            if (d.epilogue == MLVC_EPI_REGLU && k.bm % 64 != 0)
+            // Whether the variant's own kernel runs this conv. Its plan made
+            // sure, but a descriptor may have changed since (another size,
+            // epilogue, fusion or split): conv_mfma_kernel runs it then, pixel
+            // by pixel, with the same tile and packed weights.
+            // The weight-streaming kernel: a plain input, no split, whole
+            // rings of channels, no ReGLU, DEPTH_TO_SPACE(2) or none.
+            bool own = !k.ws_ic || (!a.x2 && a.s2d <= 1 && a.ksplit == 1 &&
+                                    (k.ws_mult <= 16 || d.ic % k.ws_mult == 0) &&
+                                    d.epilogue != MLVC_EPI_REGLU && a.d2s <= 2);
+            // The 1x1 kernels: as in eligible(). With all splits in one
+            // workgroup each wave multiplies whole 64-channel halves.
+            if (k.point_ic)
+                own = a.ih == 1 && d.ic % k.point_ic == 0 && a.iw % 2 == 0 && a.s2d <= 1 && a.d2s <= 1 &&
+                      (a.ksplit > 1) == k.point_split && (!a.x2 || a.ic_split % 16 == 0) && d.epilogue != MLVC_EPI_REGLU &&
+                      (!k.point_split || (!a.x2 && a.ksplit <= 8 && a.split_c % k.point_ic == 0)) &&
+                      static_cast<std::uint64_t>((d.oc + k.bm - 1) / k.bm) * k.bm * d.ic * 2 < (1ull << 31);
+            if (d.epilogue == MLVC_EPI_REGLU && k.bm % 64 != 0 && a.ksplit == 1)
                 throw std::runtime_error("conv: ReGLU needs a variant of whole 64-channel blocks");
-            const bool vec = rows && (even || k.point_ic) && halves && epilogue;
+            const bool vec = own && rows && (even || k.point_ic);
             const bool nchw = !d.in_nhwc && !d.out_nhwc;
-            const auto ragged = rows && !even && images4 && nchw && epilogue ? k.launch_rag[a.iw & 1] : nullptr;
+            const auto ragged = own && rows && !even && images4 && nchw ? k.launch_rag[a.iw & 1] : nullptr;
             a.tiles_x = (a.ow + k.tw - 1) / k.tw;
             a.nchunks = (d.ic + k.kc - 1) / k.kc;
             a.tiles = a.tiles_x * ((a.oh + k.th - 1) / k.th);
@@ -538,14 +543,11 @@ void launch_conv(const mlvc_hip_conv_desc& d, void* s)
             const std::uint64_t src_plane = static_cast<std::uint64_t>(a.ih) * a.iw * 4 * 2;
             const bool s2d_vec = k.launch_s2d && a.s2d == 2 && (reinterpret_cast<std::uintptr_t>(d.x) & 15u) == 0 &&
                                  a.iw % 8 == 0 && (static_cast<std::uint64_t>(d.ic / 4) + k.kc / 4 + 1) * src_plane < (1ull << 31);
-            if (k.ws_ic && k.ws_mult > 16 && d.ic % k.ws_mult != 0)
-                throw std::runtime_error("conv: variant does not match the geometry");
-            if (k.ws_ic && (d.x2 || a.s2d > 1)) throw std::runtime_error("conv: variant needs a plain input");
-            // Operands without the alignment: the variants the plan chooses
-            // stage them pixel by pixel (NCHW).
+            // Only the variants the plan chooses have the general kernel's
+            // build (NCHW).
             if (k.ws_ic && !vec && !ragged && (!k.launch_scalar || !nchw))
-                throw std::runtime_error(epilogue ? "conv: variant needs 16-byte row staging"
-                                                  : "conv: variant does not run the epilogue or the depth_to_space block");
+                throw std::runtime_error(own ? "conv: variant needs 16-byte row staging"
+                                             : "conv: variant does not run the conv's epilogue, fusions or split");
             (s2d_vec ? k.launch_s2d : vec ? k.launch_vec : ragged ? ragged : k.launch_scalar)(a, grid, to_stream(s));
             if (a.ksplit > 1 && !(k.point_split && vec)) {
                 ConvArgs r = a;  // the reduce works in the real output geometry
