@@ -98,8 +98,11 @@ __device__ __forceinline__ std::uint32_t pack_f16(float a0, float a1)
 // reference's select, h < 0 ? fp16(fp32(h * alpha)) : h. The product is
 // computed for both lanes unconditionally and the choice is a per-lane
 // select, so the code is straight-line (no divergent branches around the
-// multiply). For 0 <= alpha <= 1 the select equals max(h, fp16(h * alpha))
-// (rounding is monotonic; NaN and -0 keep h), one packed max.
+// multiply). For 0 < alpha <= 1 the select equals max(h, fp16(h * alpha))
+// (rounding is monotonic; NaN and -0 keep h), one packed max; not for alpha 0,
+// where -inf gives NaN.
+__host__ __device__ __forceinline__ bool leaky_max_form(float alpha) { return alpha > 0.0f && alpha <= 1.0f; }
+
 __device__ __forceinline__ std::uint32_t leaky_h2(std::uint32_t hv, float alpha, bool max_form)
 {
     const half2_t h = __builtin_bit_cast(half2_t, hv);
@@ -118,10 +121,10 @@ __device__ __forceinline__ std::uint32_t leaky_pair(float a0, float a1, float al
 }
 
 // Epilogue modes fixed at compile time: 0 none, 1 LeakyReLU with
-// 0 <= alpha <= 1 (max form), 2 LeakyReLU with any other alpha (select form).
+// 0 < alpha <= 1 (max form), 2 LeakyReLU with any other alpha (select form).
 inline int epi_mode(int epi_is_leaky, float alpha)
 {
-    return epi_is_leaky ? (alpha >= 0.0f && alpha <= 1.0f ? 1 : 2) : 0;
+    return epi_is_leaky ? (leaky_max_form(alpha) ? 1 : 2) : 0;
 }
 
 template <int MODE>

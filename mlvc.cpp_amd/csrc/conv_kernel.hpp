@@ -671,7 +671,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
             }
         return;
     }
-    const bool max_form = a.alpha >= 0.0f && a.alpha <= 1.0f;
+    const bool max_form = leaky_max_form(a.alpha);
     if (a.d2s == 2) {
 #pragma unroll
         for (int mt = 0; mt < C::MT; ++mt)

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     const int xa = ix0 - (((ix0 % 8) + 8) % 8), col_off = ix0 - xa;
     const int koff = (lane >> 5) * 8, hsel = 4 * (lane >> 5);
     const std::uint32_t hw = static_cast<std::uint32_t>(a.h) * a.w, hw2 = hw * 2u;
-    const bool max_a = a.alpha_a >= 0.0f && a.alpha_a <= 1.0f, max_b = a.alpha_b >= 0.0f && a.alpha_b <= 1.0f;
+    const bool max_a = leaky_max_form(a.alpha_a), max_b = leaky_max_form(a.alpha_b);
 
     // ---- phase A: 3x3 conv, BM = 64 --------------------------------------
     floatx16 acc[C::MTA][C::NT];

@@ -213,7 +213,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
     }
 
     // Epilogue, wave by wave: lane l holds channel l % 32, pixels 8j + 4 (l / 32) .. + 3 of a tile.
-    const bool max_form = a.alpha >= 0.0f && a.alpha <= 1.0f;
+    const bool max_form = leaky_max_form(a.alpha);
     std::uint16_t* const es = lds0 + wave * 32 * C::EROW;
     constexpr int G = C::EPX / 8, STEPS = 32 * C::NT / C::EPX;
 #pragma unroll

@@ -384,7 +384,7 @@ __global__ __launch_bounds__(C::kThreads) __attribute__((amdgpu_waves_per_eu(C::
     // Plain outputs go through an LDS [channel][pixel] tile and leave as
     // 16-byte rows; with DEPTH_TO_SPACE(2) the 4 channels of a lane are the
     // (dy, dx) block of output channel oc0/4, stored as two 4-byte pairs.
-    const bool max_form = a.alpha >= 0.0f && a.alpha <= 1.0f;
+    const bool max_form = leaky_max_form(a.alpha);
     if constexpr (C::NHWC_D2S_EPI) {
         if (a.d2s == 2 && a.out_nhwc) {
             // Channel-last DEPTH_TO_SPACE(2): conv channel ocl is output

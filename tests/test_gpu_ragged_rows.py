@@ -8,6 +8,7 @@ NaNs, so a staged element from outside the image would show.
 """
 
 import ctypes as C
+import sys
 
 import numpy as np
 import pytest
@@ -173,3 +174,29 @@ def test_unaligned_input_pointer(case):
     lib, d, wt, b, keep, shape, _ = setup(case, offset=9)
     for v in {d.variant, *(names[n] for n in COSTED if n in names)}:
         assert torch.equal(run(lib, d, wt, b, shape, v, 1).view(torch.int16), aligned.view(torch.int16))
+
+
+@pytest.mark.parametrize("case", [CASES[1], (1, 64, 5, 16, 128, 3, 1, 1, LRELU, 0, 0), (1, 64, 6, 9, 64, 3, 1, 1, LRELU, 2, 0), CASES[12],
+                                  CASES[16], (1, 64, 5, 14, 96, 1, 1, 0, LRELU, 0, 0)],
+                         ids=lambda c: "n{}_ic{}_{}x{}_oc{}_k{}s{}p{}_e{}_d{}_c{}".format(*c))
+def test_slope_zero_of_an_infinity(monkeypatch, case):
+    """LeakyReLU with slope 0 is a product: a sum past FP16's range, -inf, gives NaN on every width and variant."""
+    monkeypatch.setattr(sys.modules[__name__], "ALPHA", 0.0)
+    case = case[:8] + (LRELU,) + case[9:]
+    print(case, flush=True)
+    lib, d, wt, b, keep, shape, _ = setup(case)
+    n, ic, h, w, oc, k, s, p = case[:8]
+    wt = (wt.float() * (60000.0 / wt.abs().max().item())).half()  # sums of around 100000
+    x = keep[0][8:8 + n * ic * h * w].cpu().reshape(n, ic, h, w)
+    y = F.conv2d(x.double(), wt.double(), b.double(), stride=s, padding=p)
+    y = F.pixel_shuffle(y, 2) if case[9] else y
+    low, high, mid = y < -66000, y > 66000, (y < -1) & (y > -65000)  # away from FP16's largest value, 65504
+    assert low.any() and high.any() and mid.any()
+    buf, count = (C.c_int * 512)(), C.c_int()
+    assert lib.mlvc_hip_conv_candidates(C.byref(d), buf, 512, C.byref(count)) == 0
+    for v in buf[:count.value]:
+        for rows in (1, 0):
+            if rows == 0 and lib.mlvc_hip_conv_variant_name(v).decode().startswith("ws_"):
+                continue
+            got = run(lib, d, wt, b, shape, v, rows)
+            assert got[low].isnan().all() and (got[high] == float("inf")).all() and (got[mid] == 0).all()
