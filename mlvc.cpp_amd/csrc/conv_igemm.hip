@@ -223,14 +223,15 @@ void split_rule(const mlvc_hip_conv_desc& d, int& ksplit, int& split_c)
 }
 
 // A channel concat: the second input's pointer, or, in a descriptor planned
-// before its tensors have addresses, the split alone.
-bool concat(const mlvc_hip_conv_desc& d) { return d.x2 || d.ic_split > 0; }
+// before its tensors have addresses, a split that leaves channels on both sides
+// (channel-last inputs have none; without a second input their split is not read).
+bool concat(const mlvc_hip_conv_desc& d) { return d.x2 || (d.ic_split > 0 && d.ic_split < d.ic && !d.in_nhwc); }
 
 // The input's fusions leave its rows stageable as 16-byte segments: a plain
 // input, or a channel concat whose split falls on 8 channels.
 bool row_staged(const mlvc_hip_conv_desc& d)
 {
-    return d.in_s2d_block <= 1 && d.ic_split % 8 == 0;
+    return d.in_s2d_block <= 1 && (!concat(d) || d.ic_split % 8 == 0);
 }
 
 bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
@@ -262,7 +263,8 @@ bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
     // concat split on a 16-channel step, offsets below 2^31; no ReGLU. Its
     // split form: split convs of a plain input and up to eight splits (a wave
     // each) of whole 64-channel halves.
-    if (k.point_ic && (!flat || !flat_1x1(d) || d.ic % k.point_ic != 0 || iw % 2 != 0 || d.ic_split % 16 != 0 ||
+    if (k.point_ic && (!flat || !flat_1x1(d) || d.ic % k.point_ic != 0 || iw % 2 != 0 ||
+                       (concat(d) && d.ic_split % 16 != 0) ||
                        (d.ksplit > 1) != k.point_split ||
                        (k.point_split && (concat(d) || d.ksplit > 8 || d.split_c % k.point_ic != 0)) ||
                        d.epilogue == MLVC_EPI_REGLU || static_cast<std::uint64_t>(d.ic) * iw * 2 >= (1ull << 31) ||

@@ -134,6 +134,31 @@ def test_ragged_rows_of_channel_last_operands_are_refused():
             assert "row staging" in msg or "channel-last operands" in msg, (ic, w, stride, cl_in, cl_out, msg)
 
 
+def test_channel_split_without_a_second_input():
+    """ic_split means a concat only where it leaves channels on both sides:
+    a descriptor without a second input that gives all its channels to the
+    first, or a channel-last one, is planned as the plain conv it is."""
+    lib = mlvc_hip.device_lib()
+    for ic, h, w, oc, k, stride in ((64, 30, 40, 128, 3, 1), (128, 40, 48, 192, 3, 2), (64, 10, 14, 96, 1, 1), (72, 9, 24, 64, 3, 1),
+                                    (1024, 23, 40, 256, 1, 1)):
+        want, _ = plan(ic, h, w, oc, k, stride, pad=k // 2)
+        d, _ = plan(ic, h, w, oc, k, stride, pad=k // 2)
+        d.ic_split = ic
+        names = candidates(ic, h, w, oc, desc=want)
+        assert lib.mlvc_hip_conv_plan(C.byref(d)) == 0
+        assert (d.variant, d.vector_io) == (want.variant, want.vector_io) and candidates(ic, h, w, oc, desc=d) == names
+        # Planned before the tensors have addresses: a concat, which the
+        # weight-streaming kernel does not run.
+        d.ic_split = 32
+        assert lib.mlvc_hip_conv_plan(C.byref(d)) == 0
+        assert not any(n.startswith("ws_") for n in candidates(ic, h, w, oc, desc=d))
+        if k == 3:
+            for cl in (want, d):
+                cl.in_nhwc = 1
+            assert lib.mlvc_hip_conv_plan(C.byref(want)) == 0 and lib.mlvc_hip_conv_plan(C.byref(d)) == 0
+            assert d.variant == want.variant and lib.mlvc_hip_conv_variant_name(d.variant).decode().startswith("ws_")
+
+
 # The tuned convs of the 1920x1088 graph: (launch, ic, h, w, oc, stride,
 # DEPTH_TO_SPACE block, channel-last input, channel-last output).
 TUNED_1920 = [
