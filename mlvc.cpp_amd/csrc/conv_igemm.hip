@@ -285,15 +285,23 @@ bool eligible(const mlvc_hip_conv_desc& d, const Variant& k)
 // over random geometries of its kernel size, three inputs in turn (3x3: then
 // scaled by up to 15% where that improves the picks). The pick's distance from
 // the fastest variant, geometric mean (and by rounds of two workgroups per
-// CU, as below): 400 1x1 convs 2.4% (38%), 189 3x3 stride-1 convs 2.3% (24%),
-// 69 stride-2 ones 1.5% (19%); on 160 convs outside the fit 2.5, 2.0 and 4.2%.
+// CU, as below): 400 1x1 convs 2.4% (38%); over 1860 3x3 stride-1 and 1020
+// stride-2 convs of all kinds (shuffles of 2 and 4, batches, 3 to 512 channels,
+// channel-last operands) 3.4% and 2.6%, of aligned plain ones 3.2% and 3.6%
+// (22% and 23%). Five of the 3x3 entries were fitted on those, to mend what the
+// others missed (32->256 shuffled by 4 at 20x40: 19.9 -> 8.4 us; 256->96
+// channel-last at 179x184: 42.8 -> 27.6).
 double measured_cost(const mlvc_hip_conv_desc& d, const Variant& k, int ow, long long tiles)
 {
     const int splits = std::max(d.ksplit, 1);  // in one workgroup or in one each
     const double steps = (d.ic + 15) / 16, kk = std::ceil(steps / splits);
     const double share = static_cast<double>(tiles) * (k.point_split ? 1 : splits) / cu_count();
     const double w = k.kh == 1 ? std::max(1.0, share) : std::ceil(share);
-    const double cost = k.cost[0] + k.cost[1] * kk + w * (k.cost[2] + k.cost[3] * kk);
+    double cost = k.cost[0] + k.cost[1] * kk + w * (k.cost[2] + k.cost[3] * kk);
+    // DEPTH_TO_SPACE past 2 leaves element by element: 0.26 us for each of a
+    // thread's elements (32 at 11x24, 32->256: 13.0 us on 32 x 8x32 tiles, 8.3
+    // on 32 x 2x32).
+    if (d.out_d2s_block > 2) cost += 0.26 * k.bm * k.th * k.tw / 256;
     // 3x3 rows that are no multiple of 8: without ragged builds they are
     // staged pixel by pixel, 16 or 32 two-byte loads each, 3 to 12 times the
     // time of the row staging (256->256 stride 2 on 58x103: 213 against 18 us;

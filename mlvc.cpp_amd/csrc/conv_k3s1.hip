@@ -37,7 +37,7 @@ const Variant kTable[] = {
     MLVC_VARIANT_DB(128, 4, 64, 3, 3, 1, 16),
     MLVC_VARIANT_DB(64, 4, 64, 3, 3, 1, 16),
     costed(MLVC_VARIANT_OCC(32, 2, 64, 3, 3, 1, 16, 4), 2.179f, 0.678f, 0.959f, 0.314f),
-    MLVC_VARIANT_WO(32, 2, 32, 3, 3, 1, 16, 1, 2, 4),
+    costed(MLVC_VARIANT_WO(32, 2, 32, 3, 3, 1, 16, 1, 2, 4), 2.555f, 0.680f, 0.416f, 0.255f),
     MLVC_VARIANT_WO(64, 2, 32, 3, 3, 1, 16, 1, 2, 4),
     MLVC_VARIANT_WS(256, 4, 32, 128, 2),
     MLVC_VARIANT_WS(128, 4, 32, 128, 2),
@@ -50,7 +50,7 @@ const Variant kTable[] = {
     // 68x120 and 136x240 decoder convs run without padded columns.
     costed(with_ragged_ws<WsCfg<128, 4, 24, 64, 2, 1, 4, 9>>(MLVC_VARIANT_WSR(128, 4, 24, 64, 2, 9)), 0.773f, 0.665f, 2.488f, 0.605f),
     MLVC_VARIANT_WSR(128, 8, 24, 64, 2, 9),
-    MLVC_VARIANT_WSR(128, 4, 40, 64, 2, 9),
+    costed(with_scalar_ws<WsCfg<128, 4, 40, 64, 2, 1, 4, 9>>(MLVC_VARIANT_WSR(128, 4, 40, 64, 2, 9)), 1.685f, 0.113f, 4.052f, 1.204f),
     MLVC_VARIANT_WSR(128, 4, 48, 64, 2, 9),
     costed(with_scalar_ws<WsCfg<128, 8, 32, 64, 2>>(MLVC_VARIANT_WS(128, 8, 32, 64, 2)), 2.118f, 0.216f, 4.243f, 1.777f),
     // Two m-tiles per wave with a 9-step ring.

@@ -14,12 +14,12 @@ const Variant kTable[] = {
     MLVC_VARIANT_OCC(32, 4, 64, 3, 3, 2, 16, 4),
     MLVC_VARIANT(32, 4, 64, 3, 3, 2, 16),
     MLVC_VARIANT(64, 2, 64, 3, 3, 2, 16),
-    MLVC_VARIANT(64, 4, 32, 3, 3, 2, 16),
+    costed(MLVC_VARIANT(64, 4, 32, 3, 3, 2, 16), 1.875f, 0.785f, 1.998f, 1.064f),
     MLVC_VARIANT(64, 8, 16, 3, 3, 2, 16),
     MLVC_VARIANT(128, 2, 64, 3, 3, 2, 16),
     MLVC_VARIANT(64, 4, 32, 3, 3, 2, 32),
     MLVC_VARIANT(64, 8, 16, 3, 3, 2, 32),
-    MLVC_VARIANT_WO(32, 2, 32, 3, 3, 2, 16, 1, 2, 4),
+    costed(MLVC_VARIANT_WO(32, 2, 32, 3, 3, 2, 16, 1, 2, 4), 1.921f, 0.808f, 0.582f, 0.291f),
     MLVC_VARIANT_WO(64, 2, 32, 3, 3, 2, 16, 1, 2, 4),
     MLVC_VARIANT_WO(64, 2, 32, 3, 3, 2, 16, 2, 1, 4),
     MLVC_VARIANT_OCC(32, 2, 64, 3, 3, 2, 16, 4),
@@ -46,7 +46,7 @@ const Variant kTable[] = {
     // CU at 68x120 (255 workgroups).
     MLVC_VARIANT_WS2R(192, 4, 24, 64, 2, 6, 9),
     MLVC_VARIANT_WS2R(192, 2, 48, 64, 2, 6, 9),
-    MLVC_VARIANT_WS2R(256, 4, 8, 64, 2, 8, 9),
+    costed(with_scalar_ws<WsCfg<256, 4, 8, 64, 2, 2, 8, 9>>(MLVC_VARIANT_WS2R(256, 4, 8, 64, 2, 8, 9)), 1.232f, 0.0f, 2.734f, 1.017f),
     // Four workgroups per CU (128 registers, 29 KB of LDS each): the
     // stride-2 convs wait on memory, and more waves keep more loads in flight.
     costed(with_ragged_ws<WsCfg<128, 2, 32, 32, 4, 2, 4>>(MLVC_VARIANT_WS2(128, 2, 32, 32, 4, 4)), 1.517f, 0.811f, 2.753f, 0.270f),

@@ -159,6 +159,26 @@ def test_channel_split_without_a_second_input():
             assert d.variant == want.variant and lib.mlvc_hip_conv_variant_name(d.variant).decode().startswith("ws_")
 
 
+def test_plan_of_convs_beside_the_plain_ones():
+    """Shuffles past 2 leave element by element, so few workgroups want small
+    tiles; and the plan knows the 40- and 8-pixel-wide tiles whose widths
+    divide the plane. (Chosen otherwise, 1.5 to 2.4 times as slow.)"""
+    lib = mlvc_hip.device_lib()
+    lib.mlvc_hip_conv_variant_name.restype = C.c_char_p
+    for want, ic, h, w, oc, stride, fields in (
+            ("mfma_bm32_2x32_k3x3_s1", 32, 20, 40, 256, 1, dict(out_d2s_block=4)),
+            ("mfma_bm32_2x32_k3x3_s1", 32, 11, 24, 144, 1, dict(out_d2s_block=3)),
+            ("ws_bm128_4x40_k3x3_s1", 256, 179, 184, 96, 1, dict(in_nhwc=1, out_nhwc=1)),
+            ("ws_bm128_4x40_k3x3_s1", 256, 124, 304, 256, 1, {}),
+            ("mfma_bm32_2x32_k3x3_s2", 64, 453, 608, 32, 2, {}),
+            ("mfma_bm32_2x32_k3x3_s2", 32, 56, 80, 256, 2, {})):
+        d, _ = plan(ic, h, w, oc, stride=stride)
+        for f, v in fields.items():
+            setattr(d, f, v)
+        assert lib.mlvc_hip_conv_plan(C.byref(d)) == 0, lib.mlvc_hip_last_error()
+        assert lib.mlvc_hip_conv_variant_name(d.variant).decode().startswith(want), (ic, h, w, oc, stride, lib.mlvc_hip_conv_variant_name(d.variant))
+
+
 # The tuned convs of the 1920x1088 graph: (launch, ic, h, w, oc, stride,
 # DEPTH_TO_SPACE block, channel-last input, channel-last output).
 TUNED_1920 = [

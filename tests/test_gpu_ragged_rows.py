@@ -160,7 +160,8 @@ def test_row_staging_equals_pixel_staging(case):
 UNALIGNED = [CASES[3], CASES[12], CASES[16], (1, 96, 12, 32, 192, 3, 1, 1, LRELU, 0, 0), (1, 128, 16, 32, 256, 3, 1, 1, LRELU, 2, 0),
              (1, 64, 16, 48, 128, 3, 2, 1, RESIDUAL, 0, 0), (1, 128, 8, 16, 96, 1, 1, 0, LRELU, 0, 0)]
 COSTED = ("ws_bm128_8x32_k3x3_s1_sc64_occ2", "ws_bm256_4x32_k3x3_s1_sc32_occ2_r3_pipe", "ws_bm256_8x16_k3x3_s1_sc32_occ2_r3_pipe",
-          "ws_bm128_4x16_k3x3_s1_sc64_occ2_r18", "ws_bm64_2x32_k3x3_s1_sc64_occ4_w2_r9")
+          "ws_bm128_4x16_k3x3_s1_sc64_occ2_r18", "ws_bm64_2x32_k3x3_s1_sc64_occ4_w2_r9", "ws_bm128_4x40_k3x3_s1_sc64_occ2_r9",
+          "ws_bm256_4x8_k3x3_s2_sc64_occ2_w8_r9")
 
 
 @pytest.mark.parametrize("case", UNALIGNED, ids=lambda c: "n{}_ic{}_{}x{}_oc{}_k{}s{}p{}_e{}_d{}_c{}".format(*c))
