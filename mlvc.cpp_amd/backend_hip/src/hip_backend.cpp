@@ -245,10 +245,15 @@ public:
     // copies that are the slot's own (nothing overwrites them before the slot
     // is waited for), since the next graph writes over the encoder's outputs
     // and the decoder's inputs are in use by the one before. The device copy
-    // is about 4 us. Four 1080p frames in flight: encoder 2637 -> 2330 us,
-    // decoder 1711 -> 1385 us. A submit on its own has nothing to run under, and
-    // the hops between streams and the slower download cost 30 us of 657: it
-    // is one chain on the backend's stream.
+    // is about 4 us. A submit on its own has nothing to run under, and the hops
+    // between streams and the slower download cost 30 us of 657: it is one
+    // chain on the backend's stream. So are all submits of small frames, whose
+    // transfers are shorter than the hops. Four frames in flight, one chain
+    // and overlapped (us):
+    //            128x60  320x184 640x360 800x440 960x536 1280x728 1920x1080
+    //   KB        27       209     810    1232    1796     3250     7231
+    //   encoder  434/528 1306/1444 1034/1037 1620/1696 1752/1772 1528/1415 2541/2234
+    //   decoder  230/298  377/348  469/416  571/502  665/574  881/738 1566/1296
     void configure_codec_io(const CodecIoConfig& cfg)
     {
         if (codec_on_) fail("codec I/O is already configured");
@@ -322,6 +327,10 @@ public:
         slots_ = std::move(slots);
         codec_ = cfg;
         codec_frame_bytes_ = frame_bytes;
+        const auto& ids = encoder ? ext_out_ : ext_in_;
+        codec_slot_bytes_ = frame_bytes;
+        for (std::size_t i = 0; i < ids.size(); ++i)
+            if (encoder || static_cast<int>(i) != q) codec_slot_bytes_ += desc_bytes(desc(ids[i]));
         codec_q_ = q;
         codec_img_ = img;
         codec_encoder_ = encoder;
@@ -2381,8 +2390,11 @@ private:
     // Whether this submit's transfers may have other frames' graphs to run
     // under: other slots are in flight, or were at the previous submit (the
     // first of a burst after the last one was waited for).
+    // Not for slots of few bytes (measured at configure_codec_io; an encoder's
+    // downloads hold up the next graph's first kernels, so it needs more).
     bool pipelined()
     {
+        if (codec_slot_bytes_ < (codec_encoder_ ? std::size_t{2} << 20 : std::size_t{128} << 10)) return false;
         const bool others = std::any_of(slots_.begin(), slots_.end(), [](const CodecSlot& sl) { return sl.pending; });
         const bool before = codec_piped_;
         codec_piped_ = others;
@@ -2439,7 +2451,7 @@ private:
     bool codec_piped_ = false;
     bool codec_on_ = false, codec_encoder_ = false;
     CodecIoConfig codec_{};
-    std::size_t codec_frame_bytes_ = 0;
+    std::size_t codec_frame_bytes_ = 0, codec_slot_bytes_ = 0;  // of a frame; of all a slot's transfers
     int codec_q_ = -1, codec_img_ = -1;  // external input index of q; of x (encoder) / output index of x_hat (decoder)
     DeviceMem codec_lut_;
     std::vector<CodecSlot> slots_;

@@ -263,18 +263,17 @@ def test_run_takes_int32_control_input(pair):
 
 
 # Submits that find other slots in flight transfer on their own streams
-# through the slot's device copies; a lone submit is one chain. Any mix of the
-# two must give what frames submitted and waited for one by one give.
-@pytest.mark.parametrize("bursts", [(1, 3, 1, 4, 2), (4, 4, 1)])
-def test_bursts_equal_single_submits(pair, bursts):
-    d, bindings = pair
-    w, h, slots, total = 128, 60, 4, sum(bursts)
+# through the slot's device copies, where a slot has enough to transfer; a lone
+# submit, or one of a small frame, is one chain. Any mix must give what frames
+# submitted and waited for one by one give.
+def check_bursts(d, bindings, w, h, mw, mh, bursts):
+    slots, total = 4, sum(bursts)
     rng = np.random.default_rng(33)
     clips = [rng.integers(0, 256, O.yuv_frame_bytes(w, h), dtype=np.uint8) for _ in range(total)]
 
     def encode(pattern):
         enc = backend(d, "MLVCEncoder", bindings)
-        enc.configure_codec_io(w, h, MW, MH, padding=O.frame_padding(w, h, MW, MH), slots=slots)
+        enc.configure_codec_io(w, h, mw, mh, padding=O.frame_padding(w, h, mw, mh), slots=slots)
         enc.reset_state()
         out, k = [], 0
         for n in pattern:
@@ -290,7 +289,7 @@ def test_bursts_equal_single_submits(pair, bursts):
 
     def decode(pattern, latents):
         dec = backend(d, "MLVCDecoder", bindings)
-        dec.configure_codec_io(w, h, MW, MH, padding=O.frame_padding(w, h, MW, MH), slots=slots)
+        dec.configure_codec_io(w, h, mw, mh, padding=O.frame_padding(w, h, mw, mh), slots=slots)
         dec.reset_state()
         out, k = [], 0
         for n in pattern:
@@ -311,6 +310,19 @@ def test_bursts_equal_single_submits(pair, bursts):
         assert all(np.array_equal(x, y) for x, y in zip(a, b)), f"encoded frame {i}"
     for i, (a, b) in enumerate(zip(decode(ones, want), decode(bursts, want))):
         assert np.array_equal(a, b), f"decoded frame {i}"
+
+
+@pytest.mark.parametrize("bursts", [(1, 3, 1, 4, 2), (4, 4, 1)])
+def test_bursts_equal_single_submits(pair, bursts):
+    check_bursts(*pair, 128, 60, MW, MH, bursts)
+
+
+@pytest.mark.parametrize("bursts", [(1, 4, 1, 2), (4, 3)])
+def test_bursts_equal_single_submits_1080p(tmp_path, bursts):
+    """Transfers of 7 MB a frame, under the other frames' graphs."""
+    mlvc_hip.synth_write("codec_enc_1920x1088", tmp_path, 0)
+    mlvc_hip.synth_write("codec_dec_1920x1088", tmp_path, 0)
+    check_bursts(tmp_path, mlvc_hip.synth_bindings("codec_enc_1920x1088")[0], 1920, 1080, 1920, 1088, bursts)
 
 
 @pytest.mark.parametrize("count", [1, 15, 16, 17, 4096, 16 * 256 * 4 + 16, 99991])
