@@ -1,7 +1,8 @@
 """Groups of eight elements on any alignment: planes of a length that is no
 multiple of 8 give, element for element, what the same planes give padded to
 one (the operators are elementwise over the planes), and nothing past a
-plane's end is written. Large launches, with non-temporal accesses, too.
+plane's end is written. Large launches, with non-temporal accesses, too: the
+feature update on three channels of 9000003 pixels, both tails on one.
 """
 
 import ctypes as C
@@ -46,11 +47,13 @@ def same(ragged, padded, count, hw):
     assert (ragged[count * hw:] == 9).all() and (padded[count * p8:] == 9).all()
 
 
-# 9 million pixels of one channel: over 256 MB in the tails' first launch.
+# 9 million pixels of one channel: over 256 MB, so non-temporal, in the tails;
+# of three channels (309 MB) in the feature update, where one moves 103 MB.
 SIZES = [(1, 3, 1), (1, 3, 7), (2, 5, 9), (1, 16, 30), (1, 7, 135 * 241), (1, 1, 9000003)]
+FEATURE_SIZES = SIZES + [(1, 3, 9000003)]
 
 
-@pytest.mark.parametrize("n,c,hw", SIZES)
+@pytest.mark.parametrize("n,c,hw", FEATURE_SIZES)
 def test_feature_update(n, c, hw):
     print(n, c, hw, flush=True)
     g = torch.Generator().manual_seed(hw)

@@ -45,6 +45,13 @@ CASES = [
     (1, 48, 9, 58, 64, 1, 1, 0, RESIDUAL, 0, 0),    # 522
     (2, 64, 3, 5, 32, 1, 1, 0, CLAMP, 0, 0),
     (1, 128, 7, 18, 64, 1, 1, 0, LRELU, 0, 64),     # channel concat
+    (1, 64, 7, 11, 96, 1, 1, 0, LRELU, 0, 32),      # concats of odd planes: the second input's rows shift by a half too
+    (1, 64, 7, 11, 64, 3, 1, 1, NONE, 0, 32),
+    (1, 64, 9, 14, 64, 3, 1, 1, RESIDUAL, 0, 32),
+    (1, 77, 6, 13, 32, 3, 1, 1, LRELU, 0, 64),      # the second input's 13 channels end inside a chunk
+    (2, 77, 5, 13, 32, 3, 1, 1, LRELU, 0, 64),      # ...and its second image lies off 4 bytes: per-pixel staging
+    (2, 45, 5, 13, 64, 1, 1, 0, CLAMP, 0, 32),
+    (2, 96, 6, 13, 64, 3, 1, 1, NONE, 0, 48),       # two images, both inputs on 4 bytes
     (1, 768, 7, 11, 96, 1, 1, 0, LRELU, 0, 0),      # split K
 ]
 
