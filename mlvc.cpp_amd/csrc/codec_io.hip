@@ -270,7 +270,9 @@ __global__ __launch_bounds__(kYuvThreads) void model_to_yuv_rotated_kernel(const
 // so the next frame's small first kernels ran 76 us instead of 5 to 7 beside
 // it. With 4 workgroups and 16 KB in flight it takes 95 us and they run 12 to
 // 16. Four 1080p frames in flight, encoded / decoded, by workgroups: 2 2352 /
-// 1438 us, 4 2295 / 1351, 8 2310 / 1367, 16 2361 / 1406.
+// 1438 us, 4 2295 / 1351, 8 2310 / 1367, 16 2361 / 1406. It reaches 44 of the
+// link's 57 GB/s: graphs shorter than their download wait for it, but less than
+// they would with the download in their own chain.
 constexpr int kDownloadGroups = 4;
 
 __global__ __launch_bounds__(256) void download_kernel(const u32x4* __restrict__ src, u32x4* __restrict__ dst, size_t n16, int tail)

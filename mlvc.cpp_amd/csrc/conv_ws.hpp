@@ -575,7 +575,7 @@ constexpr Variant with_ragged_ws(Variant v)
 #define MLVC_VARIANT_WS(BM, TH, TW, SC, OCC)                                                                   \
     Variant{"ws_bm" #BM "_" #TH "x" #TW "_k3x3_s1_sc" #SC "_occ" #OCC, BM, TH, TW, 3, 3, 1, 16, nullptr,          \
             &launch_ws<WsCfg<BM, TH, TW, SC, OCC>>, nullptr, SC, WsCfg<BM, TH, TW, SC, OCC>::NHWC_OUT}
-// A ring RING k-steps deep (3 or 9): with one m-tile per wave, 9 steps of
+// A ring RING k-steps deep (3, 9 or 18): with one m-tile per wave, 9 steps of
 // fragments cover the L2 latency that 3 do not.
 #define MLVC_VARIANT_WSR(BM, TH, TW, SC, OCC, RING)                                                            \
     Variant{"ws_bm" #BM "_" #TH "x" #TW "_k3x3_s1_sc" #SC "_occ" #OCC "_r" #RING, BM, TH, TW, 3, 3, 1, 16, nullptr, \

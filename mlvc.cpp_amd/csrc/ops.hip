@@ -509,8 +509,8 @@ __global__ __launch_bounds__(kBlock) void y1_tail_kernel(mlvc_hip_y1_tail_desc d
 // Whether a launch of `bytes` streams past the caches: more than the 256 MB
 // MALL holds, so what it reads and writes is not found there by the next
 // launch either way. Non-temporal accesses then leave room for the lines still
-// to be merged: feature update of 64 channels at 544x960 (401 MB) 85 -> 80 us,
-// both tails of 96 channels at 272x480 (852 MB) 183 -> 167 us. Launches that
+// to be merged: feature update of 64 channels at 544x960 (401 MB) 85 -> 78 us,
+// both tails of 96 channels at 272x480 (852 MB) 183 -> 168 us. Launches that
 // fit keep ordinary accesses, whose results the next launch finds in the MALL.
 bool streams(std::size_t bytes) { return bytes > (std::size_t{256} << 20); }
 
