@@ -447,11 +447,13 @@ constexpr Variant point_split_variant(const char* name)
 #define MLVC_VARIANT_PTK(MT, NT) point_split_variant<PtSplitCfg<MT, NT>>("mfma_ptk_t" #MT "x" #NT)
 
 // Variant entry: weights packed with kc = 16. Operands off 16 bytes run the
-// per-pixel staging of conv_mfma_kernel on the same tile and packed weights.
+// per-pixel staging of conv_mfma_kernel on the same tile and packed weights, at
+// two waves per SIMD: with the registers of one (96->192 at 492x656 468 us, 64->96
+// at 189x456 49) few loads are in flight on a full chip; 286 and 28 so.
 template <class C>
 constexpr Variant point_variant(const char* name)
 {
-    Variant v{name, C::BM, 1, C::BN, 1, 1, 1, 16, &launch_mfma<Cfg<C::BM, 1, C::BN, 1, 1, 1, 16, 0, false, C::WM, C::WN, 1>>,
+    Variant v{name, C::BM, 1, C::BN, 1, 1, 1, 16, &launch_mfma<Cfg<C::BM, 1, C::BN, 1, 1, 1, 16, 0, false, C::WM, C::WN, 2>>,
               &launch_point<C>, nullptr};
     v.point_ic = C::SC * C::NBUF;
     return v;
